@@ -1,0 +1,144 @@
+"""The products beyond 64 rows (hip/prefill.hip pf_pgemm*) on the GPU, each
+output tile forced in turn, against plain PyTorch in 64 bits: rows and
+columns at and around the edges of the tiles, each epilogue, split folds."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+D, F, TMAX = 192, 768, 300
+
+
+@pytest.fixture(scope='module')
+def engine():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip('no GPU')
+    from vesta.gpt2 import VestaGPT2
+    from vesta.weights import GPT2Shape, RandomGPT2
+    return VestaGPT2(RandomGPT2(GPT2Shape(2, D, 3, F, vocab=203), 5), batch=1, tmax=TMAX, engine='layered')
+
+
+def _frag(A):
+    """Activations [M, K] in fragment order (hi and lo planes) as the kernels' producers write them."""
+    import torch
+    from vesta.prefill import _mtiles, frag_weights
+    M, K = A.shape
+    A = torch.cat([A, A.new_zeros(16 * _mtiles(M) - M, K)])
+    hi = A.half()
+    return torch.stack([frag_weights(hi), frag_weights(((A - hi.float()) * 2048).half())]).contiguous()
+
+
+def _unfrag(f, M, K):
+    import torch
+    from vesta.prefill import _mtiles
+    hi, lo = f.view(2, _mtiles(M), K // 32, 4, 16, 8).permute(0, 1, 4, 2, 3, 5).reshape(2, -1, K).double()
+    return (hi + lo / 2048)[:M]
+
+
+def _close(got, want, bound):
+    """|got - want| within ``bound`` (the largest error the arithmetic allows, per element)."""
+    over = ((got.double() - want).abs() / bound).max().item()
+    assert over <= 1, over
+
+
+@pytest.mark.parametrize('kernel', ['pf_pgemm128', 'pf_pgemm64', 'pf_pgemm64w', 'pf_pgemm32'])
+@pytest.mark.parametrize('M', [65, 127, 128, 129, 257])
+def test_products_match_64_bits(engine, monkeypatch, kernel, M):
+    import torch
+    from vesta import prefill as pf
+    m, e, layer, P = engine, engine._pf, 1, M
+    W = m.W
+    gen = torch.Generator(device='cuda').manual_seed(M)
+    A, G, Z = (torch.randn(M, n, generator=gen, device='cuda') for n in (D, F, D))
+
+    def plan(ks):
+        monkeypatch.setattr(pf, 'pgemm_plan', lambda *a: (kernel, ks))
+        e._plan = []
+        e._ws = None
+
+    def run():
+        p, e._plan = e._plan, []
+        e._replay(p)
+        torch.cuda.synchronize()
+        e.check()
+
+    def exact(a, name):
+        """The product, and its bound: 22-bit activations (2^-22 each) and K fp32 additions (2^-24 each) of terms
+        whose absolute values sum to s; plus rounding of the epilogue's few fp32 operations."""
+        w = W[name][layer].double()
+        s = a.double().abs() @ w.abs()
+        return a.double() @ w, s * (2.0 ** -22 + a.shape[1] * 2.0 ** -24)
+
+    bias = {n: W[n][layer].double() for n in ('qkvb', 'ob', 'fcb', 'pb')}
+    # qkv: queries in fp32, cache rows (positions 7 .. 7 + P - 1, those at or past tmax dropped) in fp16
+    plan(1)
+    t0 = 7
+    m.seek(t0)
+    m.keys.zero_(), m.vals.zero_()
+    Q = torch.empty(M, D, device='cuda')
+    e._pgemm(_frag(A), D, 'qkvw', layer, 3 * D, pf.MODE_QKV, bias=W['qkvb'][layer], out=Q, ldo=D, M=M, P=P)
+    run()
+    want, bound = exact(A, 'qkvw')
+    want, bound = want + bias['qkvb'], bound + 2.0 ** -23 * (want.abs() + 1)
+    _close(Q, want[:, :D], bound[:, :D])
+    for n, cache in ((1, m.keys), (2, m.vals)):
+        c = slice(n * D, (n + 1) * D)
+        _close(cache[0, layer, t0:t0 + M].reshape(-1, D), want[:min(M, TMAX - t0), c],
+               bound[:TMAX - t0, c] + 2.0 ** -11 * want[:TMAX - t0, c].abs() + 2.0 ** -25)
+        assert not cache[0, layer, :t0].any() and not cache[0, layer, t0 + M:].any() and not cache[0, 0].any()
+    # GELU in fragment order (another 22-bit rounding; its slope is below 1.13 and its exponential good to 2^-20)
+    out = torch.zeros(2 * 16 * pf._mtiles(M) * F, dtype=torch.float16, device='cuda')
+    e._pgemm(_frag(A), D, 'fcw', layer, F, pf.MODE_GELU, bias=W['fcb'][layer], F=out, M=M)
+    run()
+    want, bound = exact(A, 'fcw')
+    u = want + bias['fcb']
+    want = 0.5 * u * (1 + torch.tanh(0.7978845608028654 * (u + 0.044715 * u ** 3)))
+    _close(_unfrag(out, M, F), want, 1.13 * bound + 2.0 ** -20 * (u.abs() + 2.0 ** -10))
+    # residual, whole and with a split fold whose parts the next LayerNorm's launch adds
+    want, bound = exact(G, 'pw')
+    want, bound = want + bias['pb'] + Z.double(), bound + 2.0 ** -22 * (want.abs() + Z.double().abs() + 1)
+    for ks in (1, 2, 3):
+        plan(ks)
+        z = Z.clone()
+        nf = torch.zeros(2 * 16 * pf._mtiles(M) * D, dtype=torch.float16, device='cuda')
+        done = e._pgemm(_frag(G), F, 'pw', layer, D, pf.MODE_RESID, bias=W['pb'][layer], out=z, ldo=D,
+                        ln=(W['ln1w'][layer], W['ln1b'][layer], nf), M=M)
+        assert done == (ks > 1)
+        run()
+        _close(z, want, bound)
+        if done:
+            c = z.double() - z.double().mean(-1, keepdim=True)
+            y = c / torch.sqrt((c * c).mean(-1, keepdim=True) + 1e-5)      # gains 1, biases 0
+            _close(_unfrag(nf, M, D), y, 2.0 ** -18 * (y.abs() + 1))
+    # plain, with a column count no tile divides (the output head)
+    plan(1)
+    V = W['wte'].shape[0]
+    out = torch.zeros(M, V, device='cuda')
+    e._pgemm(_frag(A), D, 'wte', None, V, pf.MODE_PLAIN, out=out, ldo=V, M=M)
+    run()
+    w = W['wte'].double()
+    _close(out, A.double() @ w.t(), (A.double().abs() @ w.abs().t()) * (2.0 ** -22 + D * 2.0 ** -24))
+
+
+def test_more_than_64_rows_decode_and_prefill_like_fewer():
+    """70 rows (products in output tiles, the output head too) against the same rows in a batch of 8:
+    the same tokens where the margin is clear, logits within the engines' tolerance."""
+    import torch
+    from vesta.gpt2 import VestaGPT2
+    from vesta.weights import GPT2Shape, RandomGPT2, random_prompts
+    hf = RandomGPT2(GPT2Shape(2, D, 3, F, vocab=203), 5)
+    pr = torch.from_numpy(random_prompts(70, 9, 203, seed=3)).to('cuda', torch.int32)
+    got = []
+    for rows in (70, 8):
+        m = VestaGPT2(hf, batch=rows, tmax=32, engine='layered')
+        m.reset()
+        m.prefill(pr[:rows])
+        lg = [m.logits()[:8].clone()]
+        for _ in range(3):
+            m.x.copy_(pr[:rows, 0])
+            m.step()
+            lg.append(m.logits()[:8].clone())
+        m.check()
+        got.append(torch.stack(lg).cpu().numpy())
+    assert np.abs(got[0] - got[1]).max() < 1e-3

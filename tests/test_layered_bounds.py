@@ -112,3 +112,38 @@ def test_products_take_one_column_tile_per_block_up_to_32_rows(rows, tiles):
     ks = args.vals[4].value
     assert name == f'pf_mgemm{pf._mtiles(rows)}'
     assert grid == -(-(3 * D // 16) // tiles) * ks
+
+
+@pytest.mark.parametrize('M,N,K,split', [(m, n, k, s) for m in (65, 100, 999, 8192, 100000)
+                                         for n, k, s in ((64, 64, True), (2304, 768, False), (768, 3072, True),
+                                                         (6400, 1600, False), (1600, 6400, True))])
+def test_tiled_product_plans_are_ones_the_kernels_take(M, N, K, split):
+    """A kernel of PG_TILES, and every fold part at least one stage (two
+    k-steps) deep; unsplit where the product may not be."""
+    name, ks = pf.pgemm_plan(M, N, K, split)
+    assert name in pf.PG_TILES and 1 <= ks <= max(1, K // 64) and (split or ks == 1)
+
+
+@pytest.mark.parametrize('case', ['fold', 'activations', 'weights', 'output', 'gelu', 'columns'])
+def test_mis_sized_tiled_products_are_refused(case):
+    e = _engine(frag_numel=100 if case == 'weights' else None)
+    e.fn.update({n: None for n in pf.PG_TILES})
+    M = 70
+    kw = dict(Af=_af(M, D), K=D, wname='ow', layer=0, N=D, mode=pf.MODE_RESID, bias=torch.zeros(D),
+              out=torch.zeros(M, D), ldo=D, M=M)
+    if case == 'fold':
+        kw['K'] = D - 32
+    elif case == 'activations':
+        kw['Af'] = kw['Af'][:-1]
+    elif case == 'output':
+        kw['out'] = torch.zeros(M * D - 1)
+    elif case == 'gelu':
+        kw.update(wname='fcw', N=F, mode=pf.MODE_GELU, out=None, F=torch.zeros(2 * 80 * F - 1))
+    elif case == 'columns':
+        kw['N'] = D - 8
+    with pytest.raises(ValueError):
+        e._pgemm(**kw)
+    assert e._plan == []
+    if case == 'fold':
+        e._pgemm(**dict(kw, K=D))
+        assert e._plan[0][0] in pf.PG_TILES

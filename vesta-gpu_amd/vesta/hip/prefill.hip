@@ -1,13 +1,15 @@
 // Multi-token prefill for the GPT-2 program on gfx950: the P prompt positions
 // of all B rows go through each layer together (M = B * P rows), so the
 // projections are matrix products on the matrix cores instead of P decode
-// steps. Appended to the prelude (hip/prelude.h, VBLOCK 256) and compiled at
+// steps. With P = 1 the same launches are one step of the layered decode
+// engine. Appended to the prelude (hip/prelude.h, VBLOCK 256) and compiled at
 // run time by hipRTC.
 //
 // Row m of every activation buffer is position p = m % P of batch row
 // b = m / P, at sequence position t0 + p, t0 read from the device (the
-// model's position counter, advanced by P at the end). Activations are fp32
-// [M, width]; the key/value cache is the decode kernel's [B, L, tmax, H, 64]
+// model's position counter, advanced by P at the end). The residual and the
+// queries are fp32 [M, width]; what a product reads is in fragment order
+// (below). The key/value cache is the decode kernel's [B, L, tmax, H, 64]
 // fp16. Positions at or past tmax write no cache row and attend to rows
 // 0 .. tmax - 1 only.
 //
@@ -18,35 +20,9 @@
 // accumulated in fp32 on its own and combined at the end.
 
 #define PF_E 64                 // head width
-#define PF_TILE 64              // output tile of one block: 64 rows x 64 columns
-#define PF_BK 64                // fold chunk staged in LDS per step of a block
-#define PF_LDA (PF_BK + 8)      // LDS row pitch of staged operands in halves (16 bytes of padding)
-
-// ---------------------------------------------------------------- embedding
-// Z[m] = wte[tok[m]] + wpe[t0 + p]   (gpt2.vst Q1; ids and positions
-// clamped into their tables). One block per row, thread t on the eight
-// consecutive values 8t .. 8t + 7 (D <= 8 * 256).
-extern "C" __global__ __launch_bounds__(256) void pf_embed(const int* __restrict__ tok, int P,
-                                                            const int* __restrict__ tp,
-                                                            const vh_half* __restrict__ wte,
-                                                            const vh_half* __restrict__ wpe, float* __restrict__ Z,
-                                                            int D, int V, int npos) {
-  const int m = blockIdx.x, k8 = 8 * threadIdx.x;
-  int x = tok[m];
-  x = x < 0 ? 0 : (x >= V ? V - 1 : x);
-  int pos = *tp + m % P;
-  pos = pos < 0 ? 0 : (pos >= npos ? npos - 1 : pos);
-  if (k8 >= D) return;
-  float a[8], b[8];
-  unpack8(ld16(wte + (size_t)x * D + k8), a);
-  unpack8(ld16(wpe + (size_t)pos * D + k8), b);
-  float* z = Z + (size_t)m * D + k8;
-  *(vh_f32x4*)z = vh_f32x4{a[0] + b[0], a[1] + b[1], a[2] + b[2], a[3] + b[3]};
-  *(vh_f32x4*)(z + 4) = vh_f32x4{a[4] + b[4], a[5] + b[5], a[6] + b[6], a[7] + b[7]};
-}
 
 // ---------------------------------------------------------------- fragment order
-// The decode products (pf_mgemm*, at most 64 rows) read both operands in the
+// Every product reads both operands in the
 // order the matrix cores take them (v_mfma_f32_16x16x32_f16: lane l = 16 q + r
 // holds row r, fold positions 8 q .. 8 q + 7 of a 16 x 32 operand tile), so
 // that each operand load of a wave is one contiguous kilobyte:
@@ -68,20 +44,34 @@ __device__ __forceinline__ void pf_frag_put8(vh_half* __restrict__ F, int MT, in
   *(vh_u32x4*)(F + (size_t)MT * KT * 512 + at) = lo;
 }
 
+// The same for four values k4 .. k4 + 3 (k4 a multiple of 4; 8-byte stores):
+// what a lane holds of a product's output tile taken with the weights as the
+// row operand (four consecutive outputs of one activation row).
+__device__ __forceinline__ void pf_frag_put4(vh_half* __restrict__ F, int MT, int KT, int m, int k4, const float* v,
+                                             bool& bad) {
+  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+  h4 hi, lo;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    bad |= !(__builtin_fabsf(v[j]) <= VH_HALF_MAX);
+    hi[j] = (_Float16)v[j];
+    lo[j] = (_Float16)((v[j] - (float)hi[j]) * VH_LO_SCALE);
+  }
+  const size_t at = (((size_t)(m >> 4) * KT + (k4 >> 5)) * 64 + ((k4 >> 3) & 3) * 16 + (m & 15)) * 8 + (k4 & 7);
+  *(vh_u32x2*)(F + at) = __builtin_bit_cast(vh_u32x2, hi);
+  *(vh_u32x2*)(F + (size_t)MT * KT * 512 + at) = __builtin_bit_cast(vh_u32x2, lo);
+}
+
 // ---------------------------------------------------------------- products
-// C = A Wt^T over K (A fp32 [M, K] with row stride lda, Wt fp16 [N, K], the
-// transposed weight: row n holds output n's weights contiguously), then the
-// epilogue of `mode`:
+// C = A W over K (A [M, K] and W [N, K] in fragment order; W row n holds
+// output n's weights), then the epilogue of `mode`:
 //   0  out[m, n] = C + bias[n]                       (plain; bias optional)
 //   1  out[m, n] = (out[m, n] + C) + bias[n]          (residual add, in place)
-//   2  out[m, n] = gelu_tanh(C + bias[n])             (feed-forward widening)
+//   2  F[m, n] = gelu_tanh(C + bias[n])               (feed-forward widening, in fragment order)
 //   3  qkv: n < D -> out[m, n] (queries); D <= n < 2D -> key cache;
 //      2D <= n -> value cache, at this row's sequence position (fp16)
-// A block computes a 64 x 64 tile. The fold goes in chunks of 64 staged in
-// LDS (double-buffered: the next chunk's global loads are in flight while
-// one chunk is multiplied): A as fp16 halves (hi, and the remainder scaled by
-// 2^11), Wt as loaded. Wave w multiplies row tile w by the four column tiles,
-// hi and lo halves into separate accumulators. K is a multiple of 64.
+// Up to 64 rows the products are pf_mgemm* (waves split the fold), beyond
+// pf_pgemm* (output tiles).
 // gelu_tanh(u) = 0.5 u (1 + tanh(y)), y = 0.7978845608028654 (u + 0.044715 u^3),
 // evaluated as u / (1 + exp(-2 y)) (0.5 (1 + tanh y) is the logistic function
 // of 2 y): one exponential and one division instead of tanh; in fp32 its
@@ -92,7 +82,7 @@ __device__ __forceinline__ float pf_gelu(float u) {
   return u / (1.0f + __expf(-2.0f * y));
 }
 
-// The epilogue of one output value c = C[m, n] (modes above).
+// The epilogue of one output value c = C[m, n] (modes 0, 1 and 3).
 __device__ __forceinline__ void pf_epi(int mode, int m, int n, float c, const vh_half* __restrict__ bias, int N,
                                        float* __restrict__ out, int ldo, vh_half* __restrict__ kc,
                                        vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer,
@@ -103,8 +93,6 @@ __device__ __forceinline__ void pf_epi(int mode, int m, int n, float c, const vh
   } else if (mode == 1) {
     float* o = out + (size_t)m * ldo + n;
     *o = (*o + c) + bn;
-  } else if (mode == 2) {
-    out[(size_t)m * ldo + n] = pf_gelu(c + bn);
   } else {
     const int D = N / 3;
     const float val = c + bn;
@@ -120,137 +108,316 @@ __device__ __forceinline__ void pf_epi(int mode, int m, int n, float c, const vh
   }
 }
 
-// One chunk's global loads: thread t takes float4 f = t + 256 i of A
-// (row f / 16, columns 4 (f % 16)..+4) and 16-byte piece g = t + 256 i of Wt
-// (row g / 8, columns 8 (g % 8)..+8); rows past M or N read as zero.
-struct PfChunk {
-  vh_f32x4 a[4];
-  vh_u32x4 w[2];
+// Products of more than 64 rows. A block makes an output tile of 16 TM WM rows
+// x 16 TN WN columns; its WM x WN waves hold TM x TN tiles of 16 x 16 each, hi
+// and lo halves in separate accumulators (the weights are the instruction's
+// row operand, so a lane ends with four consecutive outputs of one activation
+// row: 16-byte residual / query stores, 8-byte fragment-order stores). The
+// fold goes through LDS in double-buffered stages. Fragment order makes every
+// global load one contiguous kilobyte and every LDS access conflict-free
+// without padding, and the halves are made once, by the activation's producer.
+// What bounds them: the matrix cores twice per product (hi and lo) at the
+// clock that load leaves; at 24576 x 2304 x 768 the 128 x 256 tile takes 192
+// us (453 TFLOP/s of the product, 906 of the matrix cores; hipBLASLt's fp16
+// product of the same operation count 171 us), where 64 x 64 tiles that
+// converted fp32 activations in every block took 380.
+// `ks` > 1 splits the fold over blocks: part p of tile t stores its sums in
+// ws[p][m][n] for pf_reduce_ln.
+//
+// Tiles go to the 8 XCDs (blockIdx % 8) in contiguous runs, within a run in
+// groups of 4 row tiles, so that the blocks resident on one XCD share their
+// operands in its L2.
+struct PfTile {
+  int part, mt0, nt0;
 };
-
-__device__ __forceinline__ void pf_chunk_load(PfChunk& c, const float* __restrict__ A, int lda,
-                                              const vh_half* __restrict__ Wt, int M, int N, int K, int m0, int n0,
-                                              int k0) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int f = t + 256 * i, row = m0 + (f >> 4), col = k0 + 4 * (f & 15);
-    c.a[i] = row < M ? *(const vh_f32x4*)(A + (size_t)row * lda + col) : vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int g = t + 256 * i, n = n0 + (g >> 3), col = k0 + 8 * (g & 7);
-    c.w[i] = n < N ? ld16(Wt + (size_t)n * K + col) : vh_u32x4{0u, 0u, 0u, 0u};
-  }
+template <int BM, int BN>
+__device__ __forceinline__ bool pf_tile(PfTile& tl, int MT, int NT, int ks) {
+  constexpr int GM = 4;
+  const int ntn = (NT + BN - 1) / BN, ntm = (MT + BM - 1) / BM, T = ntn * ntm * ks;
+  const int per = (T + 7) / 8, id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || id >= T) return false;      // grid: 8 * ceil(T / 8) blocks
+  const int tile = id % (ntn * ntm), g = tile / (GM * ntn), gm = min(GM, ntm - g * GM), in = tile - g * GM * ntn;
+  tl.part = id / (ntn * ntm);
+  tl.mt0 = (g * GM + in % gm) * BM;
+  tl.nt0 = (in / gm) * BN;
+  return true;
 }
 
-// The chunk into LDS: A rows as hi / lo fp16 halves, Wt rows as they are.
-// `bad` is raised when an A value is beyond the fp16 range (see vh_beyond_half8).
-__device__ __forceinline__ void pf_chunk_store(const PfChunk& c, vh_half* ah, vh_half* al, vh_half* wl, bool& bad) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int f = t + 256 * i, row = f >> 4, col = 4 * (f & 15);
-    const float v[4] = {c.a[i].x, c.a[i].y, c.a[i].z, c.a[i].w};
-    _Float16 h[4], l[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      bad |= !(__builtin_fabsf(v[j]) <= VH_HALF_MAX);
-      h[j] = (_Float16)v[j];
-      l[j] = (_Float16)((v[j] - (float)h[j]) * VH_LO_SCALE);
-    }
-    *(vh_u32x2*)(ah + row * PF_LDA + col) = vh_u32x2{
-        (unsigned)__builtin_bit_cast(unsigned short, h[0]) | ((unsigned)__builtin_bit_cast(unsigned short, h[1]) << 16),
-        (unsigned)__builtin_bit_cast(unsigned short, h[2]) | ((unsigned)__builtin_bit_cast(unsigned short, h[3]) << 16)};
-    *(vh_u32x2*)(al + row * PF_LDA + col) = vh_u32x2{
-        (unsigned)__builtin_bit_cast(unsigned short, l[0]) | ((unsigned)__builtin_bit_cast(unsigned short, l[1]) << 16),
-        (unsigned)__builtin_bit_cast(unsigned short, l[2]) | ((unsigned)__builtin_bit_cast(unsigned short, l[3]) << 16)};
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int g = t + 256 * i, n = g >> 3, col = 8 * (g & 7);
-    *(vh_u32x4*)(wl + n * PF_LDA + col) = c.w[i];
-  }
-}
-
-// One staged chunk (PF_BK deep) multiplied into wave `wave`'s row tile: the
-// hi and lo halves of A against the four column tiles of Wt.
-__device__ __forceinline__ void pf_chunk_mma(vh_half (*buf)[PF_TILE * PF_LDA], int wave, int r, int kq,
-                                             vh_f32x4* acc, vh_f32x4* acl) {
-#pragma unroll
-  for (int ks = 0; ks < PF_BK; ks += 32) {
-    const int k = ks + kq;
-    const vh_u32x4 ah = *(const vh_u32x4*)(buf[0] + (16 * wave + r) * PF_LDA + k);
-    const vh_u32x4 al = *(const vh_u32x4*)(buf[1] + (16 * wave + r) * PF_LDA + k);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const vh_u32x4 b = *(const vh_u32x4*)(buf[2] + (16 * j + r) * PF_LDA + k);
-      acc[j] = vh_mfma(ah, b, acc[j]);
-      acl[j] = vh_mfma(al, b, acl[j]);
-    }
-  }
-}
-
-// `ksplit` > 1 splits K over blocks as well: block b makes part b / tiles of
-// the fold for tile b % tiles and stores its partial tile in ws[part][m][n];
-// pf_reduce then adds the parts in part order and applies the epilogue.
-extern "C" __global__ __launch_bounds__(256) void pf_gemm(
-    const float* __restrict__ A, int lda, const vh_half* __restrict__ Wt, const vh_half* __restrict__ bias,
-    int M, int N, int K, int mode, float* __restrict__ out, int ldo,
-    vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L,
-    int tmax, int ksplit, float* __restrict__ ws, unsigned* __restrict__ err) {
-  __shared__ __attribute__((aligned(16))) vh_half lds[2][3][PF_TILE * PF_LDA];   // [buffer][hi, lo, Wt]
-  const int ntn = (N + PF_TILE - 1) / PF_TILE, ntm = (M + PF_TILE - 1) / PF_TILE;
-  const int tile = blockIdx.x % (ntn * ntm), kp = blockIdx.x / (ntn * ntm);
-  const int tn = tile % ntn, tm = tile / ntn;
-  const int m0 = tm * PF_TILE, n0 = tn * PF_TILE;
-  const int nch = K / PF_BK, c0 = kp * nch / ksplit, c1 = (kp + 1) * nch / ksplit;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r = lane & 15, kq = (lane >> 4) * 8;
-  vh_f32x4 acc[4], acl[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = acl[j] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  // Chunks go global -> registers -> LDS three deep: while chunk c is
-  // multiplied out of one LDS buffer, chunk c + 1 waits in registers for the
-  // other buffer and chunk c + 2 is in flight into a second register stage.
-  // (Unrolled by two so each register stage keeps its own name.)
-  PfChunk r0, r1;
+// A wave's TM x TN output tiles (from row tile mt0, column tile nt0) through
+// the epilogue of `mode`, or into ws[part] with a split fold.
+template <int TM, int TN>
+__device__ __forceinline__ void pf_pgemm_out(
+    const vh_f32x4 (&ah)[TM][TN], const vh_f32x4 (&al)[TM][TN], int mt0, int nt0, int part, int ks, int MT,
+    const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,
+    vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L, int tmax,
+    float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, q4 = 4 * (lane >> 4), t0 = mode == 3 ? *tp : 0;
   bool bad = false;
-  if (c0 < c1) {
-    pf_chunk_load(r0, A, lda, Wt, M, N, K, m0, n0, c0 * PF_BK);
-    pf_chunk_store(r0, lds[0][0], lds[0][1], lds[0][2], bad);
-  }
-  if (c0 + 1 < c1) pf_chunk_load(r0, A, lda, Wt, M, N, K, m0, n0, (c0 + 1) * PF_BK);
-  if (c0 + 2 < c1) pf_chunk_load(r1, A, lda, Wt, M, N, K, m0, n0, (c0 + 2) * PF_BK);
-  vh_lds_sync();
-  for (int c = c0; c < c1; c += 2) {
-    pf_chunk_mma(lds[0], wave, r, kq, acc, acl);
-    if (c + 1 < c1) pf_chunk_store(r0, lds[1][0], lds[1][1], lds[1][2], bad);
-    if (c + 3 < c1) pf_chunk_load(r0, A, lda, Wt, M, N, K, m0, n0, (c + 3) * PF_BK);
-    vh_lds_sync();
-    if (c + 1 >= c1) break;
-    pf_chunk_mma(lds[1], wave, r, kq, acc, acl);
-    if (c + 2 < c1) pf_chunk_store(r1, lds[0][0], lds[0][1], lds[0][2], bad);
-    if (c + 4 < c1) pf_chunk_load(r1, A, lda, Wt, M, N, K, m0, n0, (c + 4) * PF_BK);
-    vh_lds_sync();
+#pragma unroll
+  for (int a = 0; a < TM; ++a) {
+    const int m = 16 * (mt0 + a) + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+      const int n = 16 * (nt0 + b) + q4;
+      if (n >= N) continue;
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = vh_hilo(ah[a][b][j], al[a][b][j]);
+      if (ks > 1) {
+        *(vh_f32x4*)(ws + ((size_t)part * M + m) * N + n) = vh_f32x4{v[0], v[1], v[2], v[3]};
+        continue;
+      }
+      if (mode == 0) {                                  // N of any size (the output head)
+        for (int j = 0; j < 4; ++j)
+          if (n + j < N) out[(size_t)m * ldo + n + j] = bias ? v[j] + h2f(bias[n + j]) : v[j];
+        continue;
+      }
+      float bn[4];
+      unpack4(ld8(bias + n), bn);
+      if (mode == 1) {
+        float* o = out + (size_t)m * ldo + n;
+        const vh_f32x4 z = *(const vh_f32x4*)o;
+        *(vh_f32x4*)o = vh_f32x4{(z[0] + v[0]) + bn[0], (z[1] + v[1]) + bn[1], (z[2] + v[2]) + bn[2],
+                                 (z[3] + v[3]) + bn[3]};
+      } else if (mode == 2) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = pf_gelu(v[j] + bn[j]);
+        pf_frag_put4(F, MT, N / 32, m, n, v, bad);
+      } else {
+        const int D = N / 3, bi = m / P, pos = t0 + m % P;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += bn[j];
+        if (n < D) {
+          *(vh_f32x4*)(out + (size_t)m * ldo + n) = vh_f32x4{v[0], v[1], v[2], v[3]};
+        } else if (pos >= 0 && pos < tmax) {
+          const size_t at = ((size_t)(bi * L + layer) * tmax + pos) * D + (n % D);
+          *(vh_u32x2*)((n < 2 * D ? kc : vc) + at) =
+              vh_u32x2{f2h(v[0]) | ((unsigned)f2h(v[1]) << 16), f2h(v[2]) | ((unsigned)f2h(v[3]) << 16)};
+        }
+      }
+    }
   }
   if (bad) stc_u(err, VH_ERR_RANGE);
+}
+
+// Ring: NR stages of S k-steps of 32 in flight in registers before they go to
+// LDS; with WDIR the weight fragments skip LDS and go from the caches straight
+// into each wave's registers one stage ahead (the WM waves that share them
+// meet in the CU's L1).
+template <int TM, int TN, int WM, int WN, int S, bool WDIR, int NR>
+__device__ __forceinline__ void pf_pgemm_ring(
+    const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int MT, int KT, int NT, int ks,
+    const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,
+    vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L, int tmax,
+    float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {
+  constexpr int NW = WM * WN, BM = TM * WM, BN = TN * WN;
+  constexpr int FA = 2 * BM * S, FR = FA + (WDIR ? 0 : BN * S);     // fragments (1 KB) of a stage: A, all
+  constexpr int PER = FR / NW;
+  static_assert(FR % NW == 0 && (NR == 1 || NR % 2 == 0), "whole fragments per wave; stages alternate two buffers");
+  __shared__ __attribute__((aligned(16))) vh_u32x4 lds[2][FR * 64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wm = wave / WN, wn = wave % WN;
+  PfTile tl;
+  if (!pf_tile<BM, BN>(tl, MT, NT, ks)) return;
+  const int part = tl.part, mt0 = tl.mt0, nt0 = tl.nt0;
+  const int nst = KT / S, c0 = part * nst / ks, ns = (part + 1) * nst / ks - c0;     // this part's stages
+  // tiles past the last one read the last one; their sums are not stored
+  const vh_u32x4* src[PER];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int n = n0 + 16 * j + r;
-    if (n >= N) continue;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int m = m0 + 16 * wave + 4 * (lane >> 4) + v;
-      if (m >= M) continue;
-      const float cv = fmaf(acl[j][v], 1.0f / VH_LO_SCALE, acc[j][v]);
-      if (ksplit > 1)
-        ws[((size_t)kp * M + m) * N + n] = cv;
-      else
-        pf_epi(mode, m, n, cv, bias, N, out, ldo, kc, vc, P, tp, layer, L, tmax);
+  for (int i = 0; i < PER; ++i) {
+    const int f = wave * PER + i;
+    if (f < FA) {
+      const int s = f % S, t = (f / S) % BM, p = f / (S * BM);
+      src[i] = Af + ((size_t)(p * MT + min(mt0 + t, MT - 1)) * KT + c0 * S + s) * 64 + lane;
+    } else {
+      const int e = f - FA, s = e % S, t = e / S;
+      src[i] = Wf + ((size_t)min(nt0 + t, NT - 1) * KT + c0 * S + s) * 64 + lane;
     }
   }
+  vh_f32x4 ah[TM][TN], al[TM][TN];
+#pragma unroll
+  for (int a = 0; a < TM; ++a)
+#pragma unroll
+    for (int b = 0; b < TN; ++b) ah[a][b] = al[a][b] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  vh_u32x4 st[NR][PER];
+  auto gload = [&](vh_u32x4 (&d)[PER], int c) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) d[i] = src[i][(size_t)c * S * 64];
+  };
+  auto put = [&](const vh_u32x4 (&d)[PER], int buf) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) lds[buf][(wave * PER + i) * 64 + lane] = d[i];
+  };
+  const vh_u32x4* wp[TN];
+  vh_u32x4 wd[S][TN];
+  gload(st[0], 0);
+  if constexpr (WDIR) {
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+      wp[b] = Wf + ((size_t)min(nt0 + wn * TN + b, NT - 1) * KT + c0 * S) * 64 + lane;
+#pragma unroll
+      for (int s = 0; s < S; ++s) wd[s][b] = wp[b][s * 64];
+    }
+  }
+  put(st[0], 0);
+#pragma unroll
+  for (int u = 1; u <= NR; ++u)
+    if (u < ns) gload(st[u % NR], u);
+  vh_lds_sync();
+  constexpr int U = NR == 1 ? 2 : NR;
+  for (int cc = 0; cc < ns; cc += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = cc + u;
+      if (c >= ns) break;
+      const vh_u32x4* sh = lds[u & 1];
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        vh_u32x4 w[TN], x[2][TM];
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+          if constexpr (WDIR)
+            w[b] = wd[s][b];
+          else
+            w[b] = sh[(FA + (wn * TN + b) * S + s) * 64 + lane];
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int a = 0; a < TM; ++a) x[p][a] = sh[((p * BM + wm * TM + a) * S + s) * 64 + lane];
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+          for (int b = 0; b < TN; ++b) {
+            ah[a][b] = vh_mfma(w[b], x[0][a], ah[a][b]);
+            al[a][b] = vh_mfma(w[b], x[1][a], al[a][b]);
+          }
+        if constexpr (WDIR)
+          if (c + 1 < ns)
+#pragma unroll
+            for (int b = 0; b < TN; ++b) wd[s][b] = wp[b][(size_t)((c + 1) * S + s) * 64];
+      }
+      if (c + 1 < ns) {       // the buffer written here was last read before the previous barrier
+        put(st[(u + 1) % NR], (u + 1) & 1);
+        if (c + 1 + NR < ns) gload(st[(u + 1) % NR], c + 1 + NR);
+      }
+      vh_lds_sync();
+    }
+  }
+  pf_pgemm_out<TM, TN>(ah, al, mt0 + wm * TM, nt0 + wn * TN, part, ks, MT, bias, M, N, mode, out, ldo, kc, vc, P, tp,
+                       layer, L, tmax, ws, F, err);
 }
+
+// Pipe: one k-step a stage; while a stage's products run, the next stage's
+// fragments go from LDS into a second register set, the stage after that from
+// registers into LDS and the one after from the caches into registers, so no
+// wave waits for LDS between its products.
+template <int TM, int TN, int WM, int WN>
+__device__ __forceinline__ void pf_pgemm_pipe(
+    const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int MT, int KT, int NT, int ks,
+    const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,
+    vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L, int tmax,
+    float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {
+  constexpr int NW = WM * WN, BM = TM * WM, BN = TN * WN;
+  constexpr int FA = 2 * BM, FR = FA + BN;           // fragments (1 KB) of a stage: A, all
+  constexpr int PER = FR / NW;
+  static_assert(FR % NW == 0 && TM % 2 == 0, "whole fragments per wave");
+  __shared__ __attribute__((aligned(16))) vh_u32x4 lds[2][FR * 64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wm = wave / WN, wn = wave % WN;
+  PfTile tl;
+  if (!pf_tile<BM, BN>(tl, MT, NT, ks)) return;
+  const int part = tl.part, mt0 = tl.mt0, nt0 = tl.nt0;
+  const int c0 = part * KT / ks, ns = (part + 1) * KT / ks - c0;
+  const vh_u32x4* src[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int f = wave * PER + i;
+    if (f < FA) {
+      const int t = f % BM, p = f / BM;
+      src[i] = Af + ((size_t)(p * MT + min(mt0 + t, MT - 1)) * KT + c0) * 64 + lane;
+    } else {
+      src[i] = Wf + ((size_t)min(nt0 + f - FA, NT - 1) * KT + c0) * 64 + lane;
+    }
+  }
+  vh_f32x4 ah[TM][TN], al[TM][TN];
+#pragma unroll
+  for (int a = 0; a < TM; ++a)
+#pragma unroll
+    for (int b = 0; b < TN; ++b) ah[a][b] = al[a][b] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  vh_u32x4 st[PER], w[2][TN], x[2][2][TM];
+  auto gload = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) st[i] = src[i][(size_t)c * 64];
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) lds[buf][(wave * PER + i) * 64 + lane] = st[i];
+  };
+  auto frags = [&](vh_u32x4 (&wf)[TN], vh_u32x4 (&xf)[2][TM], int buf) {
+#pragma unroll
+    for (int b = 0; b < TN; ++b) wf[b] = lds[buf][(FA + wn * TN + b) * 64 + lane];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) xf[p][a] = lds[buf][(p * BM + wm * TM + a) * 64 + lane];
+  };
+  auto mma = [&](const vh_u32x4 (&wf)[TN], const vh_u32x4 (&xf)[2][TM], int a0, int a1) {
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+      if (a < a0 || a >= a1) continue;
+#pragma unroll
+      for (int b = 0; b < TN; ++b) {
+        ah[a][b] = vh_mfma(wf[b], xf[0][a], ah[a][b]);
+        al[a][b] = vh_mfma(wf[b], xf[1][a], al[a][b]);
+      }
+    }
+  };
+  gload(0);
+  put(0);
+  if (1 < ns) gload(1);
+  vh_lds_sync();
+  frags(w[0], x[0], 0);
+  if (1 < ns) put(1);
+  if (2 < ns) gload(2);
+  vh_lds_sync();
+  for (int cc = 0; cc < ns; cc += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int c = cc + u;
+      if (c >= ns) break;
+      if (c + 1 < ns) frags(w[u ^ 1], x[u ^ 1], u ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(w[u], x[u], 0, TM / 2);
+      __builtin_amdgcn_sched_barrier(0);
+      if (c + 2 < ns) {       // buffer u: its last reads were before the previous barrier
+        put(u);
+        if (c + 3 < ns) gload(c + 3);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      mma(w[u], x[u], TM / 2, TM);
+      __builtin_amdgcn_sched_barrier(0);
+      vh_lds_sync();
+    }
+  }
+  pf_pgemm_out<TM, TN>(ah, al, mt0 + wm * TM, nt0 + wn * TN, part, ks, MT, bias, M, N, mode, out, ldo, kc, vc, P, tp,
+                       layer, L, tmax, ws, F, err);
+}
+
+#define PF_PGEMM(name, threads, waves, ...)                                                                         \
+  extern "C" __global__ __launch_bounds__(threads, waves) void name(                                                \
+      const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int MT, int KT, int NT, int ks,             \
+      const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,                   \
+      vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L,      \
+      int tmax, float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {                      \
+    __VA_ARGS__(Af, Wf, MT, KT, NT, ks, bias, M, N, mode, out, ldo, kc, vc, P, tp, layer, L, tmax, ws, F, err);     \
+  }
+PF_PGEMM(pf_pgemm128, 512, 2, pf_pgemm_pipe<4, 4, 2, 4>)              // 128 x 256
+PF_PGEMM(pf_pgemm64, 512, 4, pf_pgemm_pipe<2, 2, 2, 4>)               // 64 x 128, eight waves
+PF_PGEMM(pf_pgemm64w, 256, 2, pf_pgemm_ring<2, 4, 2, 2, 1, true, 2>)  // 64 x 128, four waves
+PF_PGEMM(pf_pgemm32, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, 2>)  // 32 x 64
 
 // The parts of a split product added in part order, then the epilogue. One
 // thread per output value.
@@ -267,13 +434,13 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce(
 }
 
 // ---------------------------------------------------------------- layer norm
-// Y[i] = (X[r] - mean) / sqrt(var + 1e-5) * w + b for r = row0 + i * rstride
+// F[i] = (X[r] - mean) / sqrt(var + 1e-5) * w + b for r = row0 + i * rstride
 // (biased variance; mean and variance as sums of x / D and (x - mean)^2 / D,
 // as gpt2.vst Q2 writes them): one block per output row, D <= 8 * 256,
 // thread t holding the row's eight consecutive values 8t .. 8t + 7 (16-byte
 // loads, so a wave's load is a whole kilobyte of the row), summed per thread,
-// then over the block. With F set the row goes to F in fragment order (MT
-// m-tiles: the thread writes its own piece) instead of Y. (Thread t on values
+// then over the block. The row goes to F in fragment order (MT m-tiles: the
+// thread writes its own piece). (Thread t on values
 // t, t + 256, .., one 4-byte load each, measured slower: XL B=64 decode 4.06
 // against 3.41 ms per step with the reduction below written that way.)
 __device__ __forceinline__ void pf_ld8f(const float* p, float* v) {
@@ -281,8 +448,8 @@ __device__ __forceinline__ void pf_ld8f(const float* p, float* v) {
   v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3]; v[4] = b[0]; v[5] = b[1]; v[6] = b[2]; v[7] = b[3];
 }
 __device__ __forceinline__ void pf_norm8_out(const float* v, const float* wv, const float* bv, bool in, int D, int i,
-                                             float* __restrict__ Y, vh_half* __restrict__ F, int MT,
-                                             unsigned* __restrict__ err, float* red) {
+                                             vh_half* __restrict__ F, int MT, unsigned* __restrict__ err,
+                                             float* red) {
   const float fd = (float)D;
   float s = 0.0f;
   if (in)
@@ -299,21 +466,14 @@ __device__ __forceinline__ void pf_norm8_out(const float* v, const float* wv, co
   float y[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) y[j] = (v[j] - mean) / sd * wv[j] + bv[j];
-  const int k8 = 8 * threadIdx.x;
-  if (F == nullptr) {
-    float* yp = Y + (size_t)i * D + k8;
-    *(vh_f32x4*)yp = vh_f32x4{y[0], y[1], y[2], y[3]};
-    *(vh_f32x4*)(yp + 4) = vh_f32x4{y[4], y[5], y[6], y[7]};
-    return;
-  }
   bool bad = false;
-  pf_frag_put8(F, MT, D / 32, i, k8, y, bad);
+  pf_frag_put8(F, MT, D / 32, i, 8 * threadIdx.x, y, bad);
   if (bad) stc_u(err, VH_ERR_RANGE);
 }
 
 extern "C" __global__ __launch_bounds__(256) void pf_ln(const float* __restrict__ X, int row0, int rstride,
                                                          const vh_half* __restrict__ w, const vh_half* __restrict__ b,
-                                                         float* __restrict__ Y, int D, vh_half* __restrict__ F, int MT,
+                                                         int D, vh_half* __restrict__ F, int MT,
                                                          unsigned* __restrict__ err) {
   __shared__ float red[VNWAVE];
   const int k8 = 8 * threadIdx.x;
@@ -324,13 +484,15 @@ extern "C" __global__ __launch_bounds__(256) void pf_ln(const float* __restrict_
     unpack8(ld16(w + k8), wv);
     unpack8(ld16(b + k8), bv);
   }
-  pf_norm8_out(v, wv, bv, in, D, blockIdx.x, Y, F, MT, err, red);
+  pf_norm8_out(v, wv, bv, in, D, blockIdx.x, F, MT, err, red);
 }
 
-// pf_embed and the first layer's LayerNorm into fragment order (pf_ln) in one
-// launch for a decode pass (one position per row): one block per row, the
-// row kept in registers between the two.
-extern "C" __global__ __launch_bounds__(256) void pf_embed_ln(const int* __restrict__ tok, const int* __restrict__ tp,
+// The embedding Z[m] = wte[tok[m]] + wpe[t0 + p] (gpt2.vst Q1; ids and
+// positions clamped into their tables) and the first layer's LayerNorm of it
+// (pf_ln) in one launch: one block per row, the row kept in registers between
+// the two.
+extern "C" __global__ __launch_bounds__(256) void pf_embed_ln(const int* __restrict__ tok, int P,
+                                                               const int* __restrict__ tp,
                                                                const vh_half* __restrict__ wte,
                                                                const vh_half* __restrict__ wpe, float* __restrict__ Z,
                                                                int D, int V, int npos, const vh_half* __restrict__ w,
@@ -341,7 +503,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_embed_ln(const int* __restr
   const bool in = k8 < D;
   int x = tok[m];
   x = x < 0 ? 0 : (x >= V ? V - 1 : x);
-  int pos = *tp;
+  int pos = *tp + m % P;
   pos = pos < 0 ? 0 : (pos >= npos ? npos - 1 : pos);
   float v[8] = {}, wv[8] = {}, bv[8] = {};
   if (in) {
@@ -356,17 +518,17 @@ extern "C" __global__ __launch_bounds__(256) void pf_embed_ln(const int* __restr
     *(vh_f32x4*)z = vh_f32x4{v[0], v[1], v[2], v[3]};
     *(vh_f32x4*)(z + 4) = vh_f32x4{v[4], v[5], v[6], v[7]};
   }
-  pf_norm8_out(v, wv, bv, in, D, m, nullptr, F, MT, err, red);
+  pf_norm8_out(v, wv, bv, in, D, m, F, MT, err, red);
 }
 
 // A split residual product's parts added in part order (pf_reduce, mode 1:
 // Z[m, n] = (Z[m, n] + C) + bias[n]) and the LayerNorm that reads Z next (as
-// pf_ln, into Y or F), in one launch: one block per row, the row kept in
+// pf_ln), in one launch: one block per row, the row kept in
 // registers between the two.
 extern "C" __global__ __launch_bounds__(256) void pf_reduce_ln(
     const float* __restrict__ ws, int ksplit, const vh_half* __restrict__ bias, int M, int D,
-    float* __restrict__ Z, const vh_half* __restrict__ w, const vh_half* __restrict__ b, float* __restrict__ Y,
-    vh_half* __restrict__ F, int MT, unsigned* __restrict__ err) {
+    float* __restrict__ Z, const vh_half* __restrict__ w, const vh_half* __restrict__ b, vh_half* __restrict__ F,
+    int MT, unsigned* __restrict__ err) {
   __shared__ float red[VNWAVE];
   const int m = blockIdx.x, k8 = 8 * threadIdx.x;
   const bool in = k8 < D;
@@ -394,10 +556,10 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_ln(
     *(vh_f32x4*)zp = vh_f32x4{v[0], v[1], v[2], v[3]};
     *(vh_f32x4*)(zp + 4) = vh_f32x4{v[4], v[5], v[6], v[7]};
   }
-  pf_norm8_out(v, wv, bv, in, D, m, Y, F, MT, err, red);
+  pf_norm8_out(v, wv, bv, in, D, m, F, MT, err, red);
 }
 
-// ---------------------------------------------------------------- decode products
+// ---------------------------------------------------------------- products of few rows
 // C = A W over K for M <= 16 MT rows, both operands in fragment order (above):
 // the weights streamed from memory straight into the matrix cores' registers,
 // the activations read as they are (hi and lo planes, each multiplied into
@@ -415,18 +577,18 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_ln(
 // next k-step's weights and activations in flight. The waves' partial tiles
 // are added in LDS in wave order. Then either the part is stored (ks > 1:
 // ws[part][m][n], added by pf_reduce / pf_reduce_ln / pf_reduce_frag), or the
-// epilogue of `mode` is applied: 0, 1 and 3 as pf_epi (one position per row);
+// epilogue of `mode` is applied: 0, 1 and 3 as pf_epi;
 // 2 (GELU) writes the result in fragment order into F, as the activation of
 // the next product (N / 32 k-steps).
 #define PF_MW 8
 #define PF_WFIRST 8     // k-steps of a wave up to which all its weight fragments are loaded first
 
-// pf_epi for eight consecutive columns n .. n + 7 of row m (one position per
-// row), modes 1 (residual) and 3 (qkv: queries, or eight values of a key /
+// pf_epi for eight consecutive columns n .. n + 7 of row m (at sequence
+// position pos), modes 1 (residual) and 3 (qkv: queries, or eight values of a key /
 // value cache row as one 16-byte store); the same arithmetic per value.
 __device__ __forceinline__ void pf_epi8(int mode, int m, int n, float* v, const float* bn, const float* z, int pos,
                                         int N, float* __restrict__ out, int ldo, vh_half* __restrict__ kc,
-                                        vh_half* __restrict__ vc, int layer, int L, int tmax) {
+                                        vh_half* __restrict__ vc, int P, int layer, int L, int tmax) {
   if (mode == 1) {
     float* o = out + (size_t)m * ldo + n;
 #pragma unroll
@@ -448,7 +610,7 @@ __device__ __forceinline__ void pf_epi8(int mode, int m, int n, float* v, const 
   unsigned short h[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) h[j] = f2h(v[j]);
-  const size_t at = ((size_t)(m * L + layer) * tmax + pos) * D + (n % D);
+  const size_t at = ((size_t)(m / P * L + layer) * tmax + pos) * D + (n % D);
   *(vh_u32x4*)((n < 2 * D ? kc : vc) + at) =
       vh_u32x4{h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16), h[4] | ((unsigned)h[5] << 16),
                h[6] | ((unsigned)h[7] << 16)};
@@ -457,7 +619,7 @@ template <int MT, int MN, bool WNT>
 __device__ __forceinline__ void pf_mgemm_body(
     int vb, const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int KT, int NT, int ks,
     const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,
-    vh_half* __restrict__ kc, vh_half* __restrict__ vc, const int* __restrict__ tp, int layer, int L, int tmax,
+    vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L, int tmax,
     float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {
   __shared__ __attribute__((aligned(16))) vh_f32x4 red[PF_MW][MN * MT * 64];
   __shared__ __attribute__((aligned(16))) float tile[16 * MT][16 * MN + 4];
@@ -488,7 +650,7 @@ __device__ __forceinline__ void pf_mgemm_body(
   if (eok) {
     if (bias && mode != 2) unpack8(ld16(bias + en), eb);
     if (mode == 1) pf_ld8f(out + (size_t)em * ldo + en, ez);
-    if (mode == 3) epos = *tp;
+    if (mode == 3) epos = *tp + em % P;
   }
   // weight fragments: nontemporal (WNT) where the model's weights cannot stay
   // in the memory-side cache between steps (the host picks the kernel)
@@ -609,7 +771,7 @@ __device__ __forceinline__ void pf_mgemm_body(
         *(vh_f32x4*)p = vh_f32x4{v[0], v[1], v[2], v[3]};
         *(vh_f32x4*)(p + 4) = vh_f32x4{v[4], v[5], v[6], v[7]};
       } else {
-        pf_epi8(mode, m, n, v, eb, ez, epos, N, out, ldo, kc, vc, layer, L, tmax);     // (e is this thread's item)
+        pf_epi8(mode, m, n, v, eb, ez, epos, N, out, ldo, kc, vc, P, layer, L, tmax);     // (e is this thread's item)
       }
     }
     return;
@@ -617,7 +779,7 @@ __device__ __forceinline__ void pf_mgemm_body(
   for (int e = threadIdx.x; e < 16 * MT * 16 * MN; e += PF_MW * 64) {
     const int m = e / (16 * MN), c = e % (16 * MN), n = n0 + c;
     if (m >= M || n >= N) continue;
-    pf_epi(mode, m, n, tile[m][c], bias, N, out, ldo, kc, vc, 1, tp, layer, L, tmax);
+    pf_epi(mode, m, n, tile[m][c], bias, N, out, ldo, kc, vc, P, tp, layer, L, tmax);
   }
 }
 
@@ -625,9 +787,9 @@ __device__ __forceinline__ void pf_mgemm_body(
   extern "C" __global__ __launch_bounds__(PF_MW * 64) void name(                                                  \
       const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int KT, int NT, int ks,                    \
       const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,                 \
-      vh_half* __restrict__ kc, vh_half* __restrict__ vc, const int* __restrict__ tp, int layer, int L, int tmax, \
-      float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {                              \
-    pf_mgemm_body<MT, MN, WNT>(blockIdx.x, Af, Wf, KT, NT, ks, bias, M, N, mode, out, ldo, kc, vc, tp, layer, L,    \
+      vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L,      \
+      int tmax, float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {                              \
+    pf_mgemm_body<MT, MN, WNT>(blockIdx.x, Af, Wf, KT, NT, ks, bias, M, N, mode, out, ldo, kc, vc, P, tp, layer, L, \
                                tmax, ws, F, err);                                                                 \
   }
 PF_MGEMM(pf_mgemm1, 1, 1, false)
@@ -742,12 +904,13 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_frag(const float* __
 // across them),
 // the max-subtracted softmax (Q6), and the weighted values (Q7: eight lanes
 // per position, 8 dims each), read from the fp16 cache the qkv product just
-// wrote. O[m, h * 64 + e] receives the head's output.
+// wrote. F receives the head's output, row m, in fragment order.
 // `ws` holds each wave's scores, then weights, for up to PF_TMAX positions.
 extern "C" __global__ __launch_bounds__(256) void pf_attn(const float* __restrict__ Q, const vh_half* __restrict__ kc,
-                                                           const vh_half* __restrict__ vc, float* __restrict__ O,
-                                                           int M, int P, const int* __restrict__ tp, int layer,
-                                                           int L, int tmax, int H) {
+                                                           const vh_half* __restrict__ vc, int M, int P,
+                                                           const int* __restrict__ tp, int layer, int L, int tmax,
+                                                           int H, vh_half* __restrict__ F, int MT,
+                                                           unsigned* __restrict__ err) {
   __shared__ float ws[VNWAVE][PF_TMAX];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int item = blockIdx.x * VNWAVE + wave;
@@ -842,9 +1005,9 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn(const float* __restric
       o[j] += __shfl_xor(o[j], 32, 64);
     }
     if (a == 0) {
-      float* dst = O + (size_t)m * D + h * PF_E + 8 * b;
-      *(vh_f32x4*)dst = vh_f32x4{o[0], o[1], o[2], o[3]};
-      *(vh_f32x4*)(dst + 4) = vh_f32x4{o[4], o[5], o[6], o[7]};
+      bool bad = false;
+      pf_frag_put8(F, MT, D / 32, m, h * PF_E + 8 * b, o, bad);
+      if (bad) stc_u(err, VH_ERR_RANGE);
     }
   }
 }
@@ -864,7 +1027,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn(const float* __restric
 // caches (same box: GPT-2 small at 32 rows 0.586 -> 0.550 ms per step, the
 // attention launch 19.3 -> 17.8 us; XL at 64 rows 3.023 -> 3.000).
 extern "C" __global__ __launch_bounds__(256) void pf_attn1(const float* __restrict__ Q, const vh_half* __restrict__ kc,
-                                                            const vh_half* __restrict__ vc, float* __restrict__ O,
+                                                            const vh_half* __restrict__ vc,
                                                             const int* __restrict__ tp, int layer, int L, int tmax,
                                                             int H, vh_half* __restrict__ F, int MT,
                                                             unsigned* __restrict__ err) {
@@ -985,17 +1148,12 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1(const float* __restri
     float r = part[0][tid];
 #pragma unroll
     for (int w = 1; w < VNWAVE; ++w) r += part[w][tid];
-    if (F == nullptr)
-      O[(size_t)m * D + h * PF_E + tid] = r;
-    else
-      qs[tid] = r;
+    qs[tid] = r;
   }
-  if (F != nullptr) {       // the head's 64 outputs in fragment order, eight per thread
-    __syncthreads();
-    bool bad = false;
-    if (tid < PF_E / 8) pf_frag_put8(F, MT, D / 32, m, h * PF_E + 8 * tid, qs + 8 * tid, bad);
-    if (bad) stc_u(err, VH_ERR_RANGE);
-  }
+  __syncthreads();
+  bool bad = false;         // the head's 64 outputs in fragment order, eight per thread
+  if (tid < PF_E / 8) pf_frag_put8(F, MT, D / 32, m, h * PF_E + 8 * tid, qs + 8 * tid, bad);
+  if (bad) stc_u(err, VH_ERR_RANGE);
 }
 
 // pf_attn1 in one pass over the cache (a running softmax): lane group g
@@ -1015,7 +1173,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1(const float* __restri
 // overlaps that read and the query's; its positions beyond the step's are
 // loaded but not used.
 extern "C" __global__ __launch_bounds__(256) void pf_attn1s(const float* __restrict__ Q, const vh_half* __restrict__ kc,
-                                                             const vh_half* __restrict__ vc, float* __restrict__ O,
+                                                             const vh_half* __restrict__ vc,
                                                              const int* __restrict__ tp, int layer, int L, int tmax,
                                                              int H, vh_half* __restrict__ F, int MT,
                                                              unsigned* __restrict__ err) {
@@ -1109,17 +1267,12 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1s(const float* __restr
       r = fmaf(part[k][tid], gf[k], r);
     }
     r = r / l;
-    if (F == nullptr)
-      O[(size_t)m * D + h * PF_E + tid] = r;
-    else
-      qs[tid] = r;
+    qs[tid] = r;
   }
-  if (F != nullptr) {       // the head's 64 outputs in fragment order, eight per thread
-    __syncthreads();
-    bool bad = false;
-    if (tid < PF_E / 8) pf_frag_put8(F, MT, D / 32, m, h * PF_E + 8 * tid, qs + 8 * tid, bad);
-    if (bad) stc_u(err, VH_ERR_RANGE);
-  }
+  __syncthreads();
+  bool bad = false;         // the head's 64 outputs in fragment order, eight per thread
+  if (tid < PF_E / 8) pf_frag_put8(F, MT, D / 32, m, h * PF_E + 8 * tid, qs + 8 * tid, bad);
+  if (bad) stc_u(err, VH_ERR_RANGE);
 }
 
 // ---------------------------------------------------------------- argmax

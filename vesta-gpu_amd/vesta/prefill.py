@@ -15,14 +15,16 @@ t0 .. t0 + P - 1 written, ``x`` the token chosen after the last prompt token,
 ``t`` advanced by P, ``logits()`` that step's logits.
 
 The same launch sequence with one position per row is the layered decode
-engine (``Prefill.decode``, replayed from a captured HIP graph). Up to 64
-rows its products are ``pf_mgemm*``, which read weights packed once in the
-matrix cores' operand order (``frag_weights``) and activations that the
-LayerNorms, attention and the widening product's GELU write in that order.
+engine (``Prefill.decode``, replayed from a captured HIP graph). All products
+read weights packed once in the matrix cores' operand order
+(``frag_weights``) and activations that the LayerNorms, attention and the
+widening product's GELU write in that order: up to 64 rows ``pf_mgemm*``,
+whose waves split the fold, beyond ``pf_pgemm*`` in output tiles.
 """
 from __future__ import annotations
 
 import ctypes
+import math
 from pathlib import Path
 
 from .launch import compile_code, lib, ok, track, unload
@@ -30,25 +32,21 @@ from .launch import compile_code, lib, ok, track, unload
 PREFILL_SRC = Path(__file__).resolve().parent / 'hip' / 'prefill.hip'
 PRELUDE_SRC = Path(__file__).resolve().parent / 'hip' / 'prelude.h'
 BLOCK = 256
-TILE = 64
-CHUNK = 64                    # fold depth one product step stages in LDS
+CHUNK = 64                    # products' fold lengths are multiples of this (two 32-deep k-steps)
 HEAD = 64
-KERNELS = ('pf_embed', 'pf_ln', 'pf_gemm', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn1', 'pf_argmax_part',
-           'pf_argmax', 'pf_mgemm1', 'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n', 'pf_mgemm2n', 'pf_mgemm4n',
-           'pf_reduce_frag', 'pf_attn1s', 'pf_mhead1', 'pf_mhead2', 'pf_mhead4', 'pf_embed_ln')
+KERNELS = ('pf_ln', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn1', 'pf_argmax_part', 'pf_argmax', 'pf_mgemm1',
+           'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n', 'pf_mgemm2n', 'pf_mgemm4n', 'pf_reduce_frag', 'pf_attn1s',
+           'pf_mhead1', 'pf_mhead2', 'pf_mhead4', 'pf_embed_ln', 'pf_pgemm128', 'pf_pgemm64',
+           'pf_pgemm64w', 'pf_pgemm32')
 ARGMAX_SPLIT = 32             # blocks per row of the output-head argmax (same box, 16 -> 32: GPT-2 small 32 rows
                               # 547.6 -> 545.8 us per step, 8 rows 396.3 -> 395.5, XL 64 rows even)
-SPLIT_BLOCKS = 384            # a product with fewer output tiles than this splits its fold over blocks ...
-                              # (XL B=64 decode: 4.95 ms per step at 320-384, 5.18 at 256, 5.42 at 512)
-SPLIT_MIN_CHUNKS = 4          # ... into parts of at least this many 64-deep chunks
-FUSE_REDUCE_LN = True         # (prefill products) a split residual product's reduction makes the LayerNorm
-                              # that follows (one launch instead of two; same box, decode on these products:
-                              # GPT-2 small B=32 1.073 -> 1.055 ms per step, XL B=64 5.194 -> 5.212)
+# output tiles of the products beyond FEW_ROWS rows: 16-row tiles, 16-column tiles and waves of a block
+PG_TILES = {'pf_pgemm128': (8, 16, 8), 'pf_pgemm64': (4, 8, 8), 'pf_pgemm64w': (4, 8, 4), 'pf_pgemm32': (2, 4, 4)}
 MODE_PLAIN, MODE_RESID, MODE_GELU, MODE_QKV = 0, 1, 2, 3
-DECODE_ROWS = 64              # decode passes of up to this many rows run the fragment-order products (pf_mgemm*)
+FEW_ROWS = 64                 # products of up to this many rows are pf_mgemm*, of more pf_pgemm*
 MG_WAVES = 8                  # waves of a pf_mgemm block ...
 MG_TILES = {1: 1, 2: 1, 4: 2}  # ... and the 16-column tiles it makes, by 16-row tiles (pf_mgemm1/2/4's MN)
-MG_BLOCKS = 200               # a decode product splits its fold so that it has about this many blocks, ...
+MG_BLOCKS = 200               # such a product splits its fold so that it has about this many blocks, ...
 MG_MIN_STEPS = 16             # ... each part at least this many 32-deep k-steps (two per wave)
 MG_MIN_STEPS_LN = 8           # ... or this many for a residual product whose reduction makes the next LayerNorm
                               # (its split adds no launch; same box, 16 / 12 / 8: XL B=64 3.089 / 3.057 / 3.059
@@ -57,8 +55,6 @@ MEM_CACHE_BYTES = 256 << 20   # the device's memory-side cache: decode products 
                               # larger load them nontemporal (same box: XL B=64 3.000 -> 2.944 ms per step,
                               # medium B=16 0.958 -> 0.916; GPT-2 small's 247 MB stay in that cache between
                               # steps, nontemporal there: 32 rows 0.548 -> 0.553)
-FRAG_DECODE = True            # decode passes on the fragment-order products (else the prefill products)
-HEAD_SPLIT_N = True           # the decode pass's output head on pf_mhead* (waves split the columns)
 ATTN_ONE_PASS_BLOCKS = 1024   # decode passes with at most this many (row, head) blocks read each cache row in
                               # one pass (pf_attn1s), more in two (pf_attn1: keys, then values; fewer
                               # registers, more blocks resident). Same box, two -> one pass: small 16 / 24 rows
@@ -73,9 +69,41 @@ def supported(D, H, F):
 
 
 def _mtiles(rows: int) -> int:
-    """16-row tiles of a decode product's kernel (pf_mgemm1 / 2 / 4)."""
+    """16-row tiles of the fragment-order activations of ``rows`` rows: up to
+    64 rows those of the kernels for few rows (pf_mgemm1 / 2 / 4)."""
     t = -(-rows // 16)
-    return 1 if t <= 1 else 2 if t == 2 else 4
+    return t if t > 4 else 1 if t <= 1 else 2 if t == 2 else 4
+
+
+def pgemm_us(name, M, N, K, ks):
+    """Estimated time of a product of more than FEW_ROWS rows, in us: a fixed
+    part, and for each 32-deep k-step of a block a time by how many blocks a
+    CU gets (r). Fitted to measurements at the products of the three models
+    from 65 to 24576 rows, which it gives within about 15%; e.g. (measured,
+    us) qkv of GPT-2 small at 128 rows 6.9 / 12.4 / 27.8 in 32 x 64 / 64 x 128 /
+    128 x 256 tiles, at 1024 rows 18.4 / 18.6 / 28.3, at 24576 rows 284 / 216
+    (four waves: 189) / 192; narrowing of XL at 8192 rows 560 / 408 (384) / 336."""
+    bm, bn, _ = PG_TILES[name]
+    b = -(-M // (16 * bm)) * -(-N // (16 * bn)) * ks / 256
+    k = K / 32 / ks
+    r = math.ceil(b) if b <= 4 else b
+    if name == 'pf_pgemm128':                           # one block per CU at a time
+        us = math.ceil(b) * (11 + 0.76 * k)
+    elif name == 'pf_pgemm64':
+        us = 3.5 + k * max(0.37, 0.31 * r)
+    elif name == 'pf_pgemm64w':
+        us = 3.5 + k * max(0.50, 0.15 + 0.29 * r)
+    else:
+        us = 3 + k * max(0.165, 0.12 * r)
+    # the parts of a split fold are stored and read back
+    return us + (1 + ks * M * N * 8 / 5e6 if ks > 1 else 0)
+
+
+def pgemm_plan(M, N, K, split):
+    """Kernel and fold parts of a product of more than FEW_ROWS rows
+    (``split``: whether its fold may be split): the least ``pgemm_us``."""
+    return min(((name, ks) for name in PG_TILES for ks in ((1, 2, 3, 4, 6) if split else (1,)) if K // 64 >= 2 * ks
+                or ks == 1), key=lambda c: pgemm_us(c[0], M, N, K, c[1]))
 
 
 def frag_weights(Wt):
@@ -181,37 +209,28 @@ class Prefill:
         self._plan.append((name, self.fn[name], int(grid), _Args(vals), int(block)))
 
     def _buffers(self, M):
-        """Activation buffers for M rows (one set per row count, kept)."""
+        """Activation buffers for M rows (one set per row count, kept): the
+        residual Z, the queries Q, and the fragment-order activations AF of
+        the products over d (LayerNorm and attention outputs) and GF of the
+        one over the feed-forward width (GELU outputs). These are zeroed
+        once: rows past M are never written."""
         import torch
         if M not in self._bufs:
             m = self.m
             F = m.W['fcw'].shape[2]
+            rows = 16 * _mtiles(M)
             f32 = dict(dtype=torch.float32, device='cuda')
-            self._bufs[M] = dict(Z=torch.empty(M, m.D, **f32), A=torch.empty(M, m.D, **f32),
-                                 Q=torch.empty(M, m.D, **f32), G=torch.empty(M, F, **f32),
-                                 C=torch.empty(m.B, m.D, **f32),
+            h16 = dict(dtype=torch.float16, device='cuda')
+            self._bufs[M] = dict(Z=torch.empty(M, m.D, **f32), Q=torch.empty(M, m.D, **f32),
+                                 AF=torch.zeros(2 * rows * m.D, **h16), GF=torch.zeros(2 * rows * F, **h16),
+                                 CF=torch.zeros(2 * 16 * _mtiles(m.B) * m.D, **h16),
                                  tok=torch.empty(M, dtype=torch.int32, device='cuda'),
                                  apv=torch.empty(m.B * ARGMAX_SPLIT, **f32),
                                  api=torch.empty(m.B * ARGMAX_SPLIT, dtype=torch.int32, device='cuda'))
         return self._bufs[M]
 
-    def _decode_buffers(self, B):
-        """Fragment-order activations of a decode pass of B rows: AF for the
-        products over d (LayerNorm and attention outputs), GF for the one over
-        the feed-forward width (GELU outputs). Zeroed once: rows past B are
-        never written."""
-        import torch
-        key = ('frag', B)
-        if key not in self._bufs:
-            m = self.m
-            rows = 16 * _mtiles(B)
-            F = m.W['fcw'].shape[2]
-            h16 = dict(dtype=torch.float16, device='cuda')
-            self._bufs[key] = dict(AF=torch.zeros(2 * rows * m.D, **h16), GF=torch.zeros(2 * rows * F, **h16))
-        return self._bufs[key]
-
     def _frag(self, name):
-        """Weight ``name`` in the decode products' fragment order
+        """Weight ``name`` in the products' fragment order
         ([L,] n-tile, k-step, lane, 8; see hip/prefill.hip), made on first use
         and held. Layer weights are stored [L, in, out]; the output head
         ``wte`` [V, d] is already [out, in] and gets zero rows up to a
@@ -222,8 +241,8 @@ class Prefill:
             self._own[key] = frag_weights(W) if name == 'wte' else frag_weights(W.transpose(1, 2))
         return self._own[key]
 
-    def _mgemm(self, Af, K, wname, layer, N, mode, bias=None, out=None, ldo=0, F=None, ln=None, M=1):
-        """One decode product (``pf_mgemm*``) over M rows: A in fragment order
+    def _mgemm(self, Af, K, wname, layer, N, mode, bias=None, out=None, ldo=0, F=None, ln=None, M=1, P=1):
+        """One product of at most 64 rows (``pf_mgemm*``) over M rows (P positions each of M / P rows): A in fragment order
         (Af), weights ``wname`` (layer ``layer``) in fragment order. With a
         split fold the parts are added by a second launch: ``pf_reduce_ln``
         for a residual product followed by the LayerNorm ``ln`` = (w, b, F_out)
@@ -232,6 +251,8 @@ class Prefill:
         m = self.m
         KT, NT = K // 32, -(-N // 16)
         mt = _mtiles(M)
+        if K % 32 or M > 16 * mt or mt > 4:
+            raise ValueError(f'decode product: K={K} must be a multiple of 32 and M={M} at most 64')
         nb = -(-NT // MG_TILES[mt])
         steps = MG_MIN_STEPS_LN if mode == MODE_RESID and ln is not None else MG_MIN_STEPS
         ks = max(1, min(round(MG_BLOCKS / nb), KT // steps))
@@ -239,15 +260,13 @@ class Prefill:
         Wf = self._frag(wname)
         Wf = Wf[layer] if layer is not None else Wf
         # the extents pf_mgemm* indexes, checked before the launch is recorded
-        if K % 32 or M > 16 * mt or mt > 4:
-            raise ValueError(f'decode product: K={K} must be a multiple of 32 and M={M} at most 64')
         if Af.numel() < 2 * 16 * mt * K or Wf.numel() < NT * KT * 512:
             raise ValueError(f'decode product {wname}: operands smaller than {M}x{K} activations / {N}x{K} weights')
         if mode == MODE_GELU and (N % 32 or F is None or F.numel() < 2 * 16 * mt * N):
             raise ValueError(f'decode product {wname}: GELU output needs a fragment buffer of {M}x{N}, N % 32 == 0')
         if mode in (MODE_PLAIN, MODE_RESID, MODE_QKV) and out.numel() < M * ldo:
             raise ValueError(f'decode product {wname}: output smaller than {M} rows of {ldo}')
-        t_args = [_p(m.keys), _p(m.vals), _p(m.t), _i(layer or 0), _i(m.L), _i(m.tmax)]
+        t_args = [_p(m.keys), _p(m.vals), _i(P), _p(m.t), _i(layer or 0), _i(m.L), _i(m.tmax)]
         self._launch(f'pf_mgemm{mt}' + ('n' if self._weights_nt() else ''), nb * ks,
                      [_p(Af), _p(Wf), _i(KT), _i(NT), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out), _i(ldo)]
                      + t_args + [_p(ws), _p(F), _p(self.err)], block=MG_WAVES * 64)
@@ -255,17 +274,55 @@ class Prefill:
             return False
         if mode == MODE_RESID and ln is not None:
             w, b, Fo = ln
-            self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _p(w), _p(b), _p(None),
-                                             _p(Fo), _i(mt), _p(self.err)])
+            self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _p(w), _p(b), _p(Fo),
+                                             _i(mt), _p(self.err)])
             return True
         if mode == MODE_GELU:
             self._launch('pf_reduce_frag', -(-M * (N // 8) // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(F),
                                                                        _i(mt), _p(self.err)])
         else:
             self._launch('pf_reduce', -(-M * N // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out),
-                                                            _i(ldo), _p(m.keys), _p(m.vals), _i(1), _p(m.t),
-                                                            _i(layer or 0), _i(m.L), _i(m.tmax)])
+                                                            _i(ldo)] + t_args)
         return False
+
+    def _pgemm(self, Af, K, wname, layer, N, mode, bias=None, out=None, ldo=0, F=None, ln=None, M=1, P=1):
+        """One product of any number of rows (``pf_pgemm*``), as ``_mgemm``;
+        only a residual product with a LayerNorm after it splits its fold
+        (its reduction adds no launch)."""
+        m = self.m
+        KT, NT, MT = K // 32, -(-N // 16), _mtiles(M)
+        split = mode == MODE_RESID and ln is not None and ldo == N
+        name, ks = pgemm_plan(M, N, K, split)
+        ws = self._workspace(ks * M * N) if ks > 1 else None
+        Wf = self._frag(wname)
+        Wf = Wf[layer] if layer is not None else Wf
+        # the extents pf_pgemm* indexes, checked before the launch is recorded
+        if K % 64 or MT * 16 < M:
+            raise ValueError(f'product {wname}: K={K} must be a multiple of 64')
+        if Af.numel() < 2 * 16 * MT * K or Wf.numel() < NT * KT * 512:
+            raise ValueError(f'product {wname}: operands smaller than {M}x{K} activations / {N}x{K} weights')
+        if mode == MODE_GELU and (N % 32 or F is None or F.numel() < 2 * 16 * MT * N):
+            raise ValueError(f'product {wname}: GELU output needs a fragment buffer of {M}x{N}, N % 32 == 0')
+        if mode != MODE_GELU and out.numel() < (M - 1) * ldo + (N // 3 if mode == MODE_QKV else N):
+            raise ValueError(f'product {wname}: output smaller than {M} rows of {ldo}')
+        if mode != MODE_PLAIN and (N % 64 or ldo % 4 or bias is None):
+            raise ValueError(f'product {wname}: N={N} must be a multiple of 64, the output pitch of 4, with a bias')
+        bm, bn, waves = PG_TILES[name]
+        tiles = -(-MT // bm) * -(-NT // bn) * ks
+        self._launch(name, 8 * -(-tiles // 8),
+                     [_p(Af), _p(Wf), _i(MT), _i(KT), _i(NT), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out),
+                      _i(ldo), _p(m.keys), _p(m.vals), _i(P), _p(m.t), _i(layer or 0), _i(m.L), _i(m.tmax), _p(ws),
+                      _p(F), _p(self.err)], block=waves * 64)
+        if ks > 1:
+            w, b, Fo = ln
+            self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _p(w), _p(b), _p(Fo),
+                                             _i(MT), _p(self.err)])
+        return ks > 1
+
+    def _product(self, *a, M, **kw):
+        """A product on the kernels for its row count (True: the LayerNorm
+        that follows it is done)."""
+        return (self._mgemm if M <= FEW_ROWS else self._pgemm)(*a, M=M, **kw)
 
     def _weights_nt(self):
         """Whether the decode products load their weights nontemporal
@@ -287,87 +344,9 @@ class Prefill:
         self._launch(f'pf_mhead{mt}', -(-NT // (2 * MG_WAVES)),
                      [_p(Af), _p(Wf), _i(KT), _i(NT), _i(M), _i(N), _p(out), _i(N)], block=MG_WAVES * 64)
 
-    def _build_decode(self, buf, B, tok):
-        """One decode pass (one position per row, B <= DECODE_ROWS) on the
-        fragment-order products: LayerNorm and attention write their outputs
-        as the next product's fragment-order activations, the widening
-        product writes its GELU outputs as the narrowing one's."""
-        m = self.m
-        D, H, L = m.D, m.H, m.L
-        F = m.W['fcw'].shape[2]
-        V = m.W['wte'].shape[0]
-        W = m.W
-        mt = _mtiles(B)
-        Z, Q = buf['Z'], buf['Q']
-        fb = self._decode_buffers(B)
-        AF, GF = fb['AF'], fb['GF']
-        err = self.err
-        self._launch('pf_embed_ln', B, [_p(tok), _p(m.t), _p(W['wte']), _p(W['wpe']), _p(Z), _i(D), _i(V),
-                                        _i(W['wpe'].shape[0]), _p(W['ln1w'][0]), _p(W['ln1b'][0]), _p(AF), _i(mt),
-                                        _p(err)])
-        for layer in range(L):
-            def lw(name, layer=layer):
-                return W[name][layer]
-            self._mgemm(AF, D, 'qkvw', layer, 3 * D, MODE_QKV, bias=lw('qkvb'), out=Q, ldo=D, M=B)
-            self._launch(self._attn1(), B * H, [_p(Q), _p(m.keys), _p(m.vals), _p(None), _p(m.t), _i(layer),
-                                                _i(L), _i(m.tmax), _i(H), _p(AF), _i(mt), _p(err)])
-            if not self._mgemm(AF, D, 'ow', layer, D, MODE_RESID, bias=lw('ob'), out=Z, ldo=D,
-                               ln=(lw('ln2w'), lw('ln2b'), AF), M=B):
-                self._launch('pf_ln', B, [_p(Z), _i(0), _i(1), _p(lw('ln2w')), _p(lw('ln2b')), _p(None), _i(D),
-                                          _p(AF), _i(mt), _p(err)])
-            self._mgemm(AF, D, 'fcw', layer, F, MODE_GELU, bias=lw('fcb'), F=GF, M=B)
-            nw, nb_ = (lw('ln1w', layer + 1), lw('ln1b', layer + 1)) if layer + 1 < L else (W['lnfw'], W['lnfb'])
-            if not self._mgemm(GF, F, 'pw', layer, D, MODE_RESID, bias=lw('pb'), out=Z, ldo=D, ln=(nw, nb_, AF),
-                               M=B):
-                self._launch('pf_ln', B, [_p(Z), _i(0), _i(1), _p(nw), _p(nb_), _p(None), _i(D), _p(AF), _i(mt),
-                                          _p(err)])
-        logit, nxt = m.logits(), m.next()
-        if HEAD_SPLIT_N:
-            self._mhead(AF, D, V, logit, B)
-        else:
-            self._mgemm(AF, D, 'wte', None, V, MODE_PLAIN, out=logit, ldo=V, M=B)
-        self._launch('pf_argmax_part', B * ARGMAX_SPLIT, [_p(logit), _i(V), _i(ARGMAX_SPLIT), _p(buf['apv']),
-                                                           _p(buf['api'])])
-        self._launch('pf_argmax', B, [_p(buf['apv']), _p(buf['api']), _i(ARGMAX_SPLIT), _p(m.x), _p(nxt), _p(m.t),
-                                      _i(1)])
-
     def _attn1(self):
         """The decode attention kernel for this model's rows and heads."""
         return 'pf_attn1s' if self.m.B * self.m.H <= ATTN_ONE_PASS_BLOCKS else 'pf_attn1'
-
-    def _transposed(self, name):
-        """The weight copy ``name`` (``<w>__t``: [L, out, in]); the decode
-        kernel's own when it binds one, else made here. Held here from first
-        use on, so launch plans never point at freed memory."""
-        if name not in self._own:
-            packed = getattr(self.m.k, '_packed', {})
-            self._own[name] = packed[name] if name in packed else \
-                self.m.W[name[:-3]].transpose(-1, -2).contiguous()
-        return self._own[name]
-
-    def _gemm(self, A, lda, Wt, bias, M, N, K, mode, out, ldo, layer=0, P=1, ln=None):
-        """One product launch; with few output tiles, or a long fold, the fold
-        is split over blocks too (partial tiles into a workspace, then
-        ``pf_reduce`` adds them in order and applies the epilogue). ``ln``
-        (w, b, Y) for a residual product: the LayerNorm of all M rows of
-        ``out`` into Y that comes next; a split product then does it in the
-        launch that adds its parts (``pf_reduce_ln``). Returns whether it did."""
-        m = self.m
-        tiles = -(-M // TILE) * -(-N // TILE)
-        ks = max(1, min(-(-SPLIT_BLOCKS // tiles), (K // CHUNK) // SPLIT_MIN_CHUNKS))
-        ws = self._workspace(ks * M * N) if ks > 1 else None
-        tail = [_p(m.keys), _p(m.vals), _i(P), _p(m.t), _i(layer), _i(m.L), _i(m.tmax)]
-        self._launch('pf_gemm', tiles * ks, [_p(A), _i(lda), _p(Wt), _p(bias), _i(M), _i(N), _i(K), _i(mode),
-                                             _p(out), _i(ldo)] + tail + [_i(ks), _p(ws), _p(self.err)])
-        if FUSE_REDUCE_LN and ks > 1 and ln is not None and mode == MODE_RESID and ldo == N:
-            w, b, Y = ln
-            self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _p(w), _p(b), _p(Y),
-                                             _p(None), _i(0), _p(self.err)])
-            return True
-        if ks > 1:
-            self._launch('pf_reduce', -(-M * N // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _i(mode),
-                                                            _p(out), _i(ldo)] + tail)
-        return False
 
     def _workspace(self, n):
         """Partial tiles of split products: one buffer, grown to the largest
@@ -449,50 +428,55 @@ class Prefill:
         return g
 
     def _build(self, buf, B, P, tok):
-        if P == 1 and B <= DECODE_ROWS and FRAG_DECODE:
-            return self._build_decode(buf, B, tok)
+        """The launches of one pass: B rows of P positions each (P = 1: a
+        decode step). LayerNorm and attention write their outputs as the next
+        product's fragment-order activations (AF), the widening product its
+        GELU outputs as the narrowing one's (GF)."""
         m = self.m
         M, D, H, L = B * P, m.D, m.H, m.L
         F = m.W['fcw'].shape[2]
         V = m.W['wte'].shape[0]
         W = m.W
-        Z, A, Q, G, C = buf['Z'], buf['A'], buf['Q'], buf['G'], buf['C']
-        self._launch('pf_embed', M, [_p(tok), _i(P), _p(m.t), _p(W['wte']), _p(W['wpe']), _p(Z), _i(D), _i(V),
-                                     _i(W['wpe'].shape[0])])
-        normed = False                  # A holds LN1 of Z already (made by the last product's reduction)
+        Z, Q, AF, GF, err = buf['Z'], buf['Q'], buf['AF'], buf['GF'], self.err
+        mt = _mtiles(M)
+
+        def norm(w, b, to, rows, row0=0, stride=1):
+            self._launch('pf_ln', rows, [_p(Z), _i(row0), _i(stride), _p(w), _p(b), _i(D), _p(to), _i(_mtiles(rows)),
+                                         _p(err)])
+        self._launch('pf_embed_ln', M, [_p(tok), _i(P), _p(m.t), _p(W['wte']), _p(W['wpe']), _p(Z), _i(D), _i(V),
+                                        _i(W['wpe'].shape[0]), _p(W['ln1w'][0]), _p(W['ln1b'][0]), _p(AF), _i(mt),
+                                        _p(err)])
         for layer in range(L):
             def lw(name, layer=layer):
                 return W[name][layer]
-
-            def lt(name):
-                return self._transposed(name)[layer]
-            if not normed:
-                self._launch('pf_ln', M, [_p(Z), _i(0), _i(1), _p(lw('ln1w')), _p(lw('ln1b')), _p(A), _i(D),
-                                          _p(None), _i(0), _p(self.err)])
-            self._gemm(A, D, lt('qkvw__t'), lw('qkvb'), M, 3 * D, D, MODE_QKV, Q, D, layer, P)
-            if P == 1:      # a decode pass: a block per (row, head) (GPT-2 small, 32 rows, 1024
-                            # positions: 1.32 -> 1.07 ms per step against a wave per (row, head))
-                self._launch(self._attn1(), M * H, [_p(Q), _p(m.keys), _p(m.vals), _p(A), _p(m.t), _i(layer),
-                                                    _i(L), _i(m.tmax), _i(H), _p(None), _i(0), _p(self.err)])
+            self._product(AF, D, 'qkvw', layer, 3 * D, MODE_QKV, bias=lw('qkvb'), out=Q, ldo=D, M=M, P=P)
+            cache = [_p(Q), _p(m.keys), _p(m.vals)]
+            if P == 1:          # a block per (row, head) (GPT-2 small, 32 rows, 1024 positions:
+                                # 1.32 -> 1.07 ms per step against a wave per (row, head))
+                self._launch(self._attn1(), B * H, cache + [_p(m.t), _i(layer), _i(L), _i(m.tmax), _i(H), _p(AF),
+                                                            _i(mt), _p(err)])
             else:
                 self._launch('pf_attn', -(-M * H // (BLOCK // 64)),
-                             [_p(Q), _p(m.keys), _p(m.vals), _p(A), _i(M), _i(P), _p(m.t), _i(layer), _i(L),
-                              _i(m.tmax), _i(H)])
-            if not self._gemm(A, D, lt('ow__t'), lw('ob'), M, D, D, MODE_RESID, Z, D,
-                              ln=(lw('ln2w'), lw('ln2b'), A)):
-                self._launch('pf_ln', M, [_p(Z), _i(0), _i(1), _p(lw('ln2w')), _p(lw('ln2b')), _p(A), _i(D),
-                                          _p(None), _i(0), _p(self.err)])
-            self._gemm(A, D, lt('fcw__t'), lw('fcb'), M, F, D, MODE_GELU, G, F)
-            if layer + 1 < L:
-                nxt = (lw('ln1w', layer + 1), lw('ln1b', layer + 1), A)
-            else:
-                nxt = (W['lnfw'], W['lnfb'], C) if P == 1 else None   # the final norm: each row's last position
-            normed = self._gemm(G, F, lt('pw__t'), lw('pb'), M, D, F, MODE_RESID, Z, D, ln=nxt)
-        if not normed:
-            self._launch('pf_ln', B, [_p(Z), _i(P - 1), _i(P), _p(W['lnfw']), _p(W['lnfb']), _p(C), _i(D),
-                                      _p(None), _i(0), _p(self.err)])
+                             cache + [_i(M), _i(P), _p(m.t), _i(layer), _i(L), _i(m.tmax), _i(H), _p(AF), _i(mt),
+                                      _p(err)])
+            if not self._product(AF, D, 'ow', layer, D, MODE_RESID, bias=lw('ob'), out=Z, ldo=D,
+                                 ln=(lw('ln2w'), lw('ln2b'), AF), M=M):
+                norm(lw('ln2w'), lw('ln2b'), AF, M)
+            self._product(AF, D, 'fcw', layer, F, MODE_GELU, bias=lw('fcb'), F=GF, M=M)
+            last = layer + 1 == L
+            nxt = (W['lnfw'], W['lnfb'], AF) if last else (lw('ln1w', layer + 1), lw('ln1b', layer + 1), AF)
+            normed = self._product(GF, F, 'pw', layer, D, MODE_RESID, bias=lw('pb'), out=Z, ldo=D,
+                                   ln=nxt if P == 1 or not last else None, M=M)
+            if not normed and not (last and P > 1):
+                norm(*nxt, M)
+        if P > 1:               # the final norm: each row's last position
+            norm(W['lnfw'], W['lnfb'], buf['CF'], B, P - 1, P)
         logit, nxt = m.logits(), m.next()
-        self._gemm(C, D, W['wte'], None, B, V, D, MODE_PLAIN, logit, V)
+        head = buf['CF'] if P > 1 else AF
+        if B <= FEW_ROWS:
+            self._mhead(head, D, V, logit, B)
+        else:
+            self._pgemm(head, D, 'wte', None, V, MODE_PLAIN, out=logit, ldo=V, M=B)
         self._launch('pf_argmax_part', B * ARGMAX_SPLIT, [_p(logit), _i(V), _i(ARGMAX_SPLIT), _p(buf['apv']),
                                                            _p(buf['api'])])
         self._launch('pf_argmax', B, [_p(buf['apv']), _p(buf['api']), _i(ARGMAX_SPLIT), _p(m.x), _p(nxt), _p(m.t),
