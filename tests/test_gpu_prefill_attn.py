@@ -1,0 +1,103 @@
+"""The prefill attention kernels (hip/prefill.hip pf_attn, pf_attn16) on the
+GPU, each forced, against plain PyTorch in 64 bits: query counts and start
+positions around the edges of their tiles, cache rows past the last position
+that hold infinities and NaN, queries of extreme magnitude, and a key row with
+an infinity."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+H, TMAX, L, B = 3, 330, 2, 2
+D = 64 * H
+
+
+@pytest.fixture(scope='module')
+def engine():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip('no GPU')
+    from vesta.gpt2 import VestaGPT2
+    from vesta.weights import GPT2Shape, RandomGPT2
+    return VestaGPT2(RandomGPT2(GPT2Shape(L, D, H, 4 * D, vocab=203), 5), batch=1, tmax=32, engine='layered')._pf
+
+
+def _run(e, kernel, Q, k, v, t0, P):
+    import torch
+    from vesta import prefill as pf
+    M, MT = Q.shape[0], pf._mtiles(Q.shape[0])
+    F = torch.zeros(2 * 16 * MT * D, dtype=torch.float16, device='cuda')
+    t = torch.full((1,), t0, dtype=torch.int32, device='cuda')
+    blocks = B * H * -(-P // (16 if kernel == 'pf_attn16' else 64))
+    e._plan = []
+    p, i = pf._p, pf._i
+    e._launch(kernel, 8 * -(-blocks // 8), [p(Q), p(k), p(v), i(B), i(P), p(t), i(1), i(L), i(TMAX), i(H), p(F), i(MT),
+                                            p(e.err)])
+    plan, e._plan = e._plan, []
+    e._replay(plan)
+    torch.cuda.synchronize()
+    hi, lo = F.view(2, MT, D // 32, 4, 16, 8).permute(0, 1, 4, 2, 3, 5).reshape(2, -1, D).double()
+    return (hi + lo / 2048)[:M].view(B, P, H, 64)
+
+
+def _inputs(P, t0, scale=1.0):
+    import torch
+    gen = torch.Generator(device='cuda').manual_seed(1000 * P + t0)
+    Q = torch.randn(B * P, D, generator=gen, device='cuda') * scale
+    k, v = (torch.randn(B, L, TMAX, H, 64, generator=gen, device='cuda').half() for _ in range(2))
+    return Q, k, v
+
+
+def _check(got, Q, k, v, t0, P):
+    """Against 64 bits. A score's error is that of 22-bit queries and 64 fp32 additions, relative to the sum of its
+    terms' magnitudes; the output's is twice the largest score error (numerator and sum), the 22-bit weights and n fp32
+    additions of each, relative to the largest value."""
+    import torch
+    q = Q.view(B, P, H, 64).double().permute(0, 2, 1, 3)
+    n = t0 + P
+    K, V = (c[:, 1, :n].double().permute(0, 2, 1, 3) for c in (k, v))
+    s = q @ K.transpose(2, 3).contiguous() / 8
+    later = torch.ones(P, n, dtype=torch.bool, device='cuda').triu(t0 + 1)
+    s = s.masked_fill(later, -torch.inf)
+    want = (torch.softmax(s, -1) @ V).permute(0, 2, 1, 3)
+    ds = (q.abs() @ K.nan_to_num(0, 0, 0).abs().transpose(2, 3).contiguous()).max().item() / 8 * (2.0 ** -22 + 2.0 ** -18)
+    bound = V.abs().max().item() * (2 * ds + 2.0 ** -21 + 2 * n * 2.0 ** -24)
+    assert (got - want).abs().max().item() <= bound
+
+
+@pytest.mark.parametrize('kernel', ['pf_attn', 'pf_attn16'])
+@pytest.mark.parametrize('P', [2, 8, 15, 16, 17, 63, 64, 65, 130])
+def test_prefill_attention_matches_64_bits(engine, kernel, P):
+    for t0 in (0, 1, 62, 64, 200):
+        Q, k, v = _inputs(P, t0)
+        k[:, :, t0 + P:], v[:, :, t0 + P:] = float('nan'), float('inf')      # rows no query may see
+        _check(_run(engine, kernel, Q, k, v, t0, P), Q, k, v, t0, P)
+    engine.check()
+
+
+@pytest.mark.parametrize('kernel', ['pf_attn', 'pf_attn16'])
+def test_prefill_attention_takes_any_query_magnitude(engine, kernel):
+    import torch
+    P, t0 = 20, 70
+    for scale in (1e-30, 1e-6, 1e-3):
+        Q, k, v = _inputs(P, t0, scale)
+        _check(_run(engine, kernel, Q, k, v, t0, P), Q, k, v, t0, P)
+    # far beyond the fp16 range: the softmax is one position's
+    Q, k, v = _inputs(P, t0, 1e6)
+    got = _run(engine, kernel, Q, k, v, t0, P)
+    q0 = Q.view(B, P, H, 64)[:, 0].double()                                        # the first query of each row
+    best = torch.einsum('bhd,bshd->bhs', q0.cpu(), k[:, 1, :t0 + 1].double().cpu()).argmax(-1)
+    for b in range(B):
+        for h in range(H):
+            assert (got[b, 0, h] - v[b, 1, best[b, h], h].double()).abs().max().item() < 1e-5
+    engine.check()
+
+
+@pytest.mark.parametrize('kernel', ['pf_attn', 'pf_attn16'])
+def test_a_key_of_minus_infinite_score_has_no_weight(engine, kernel):
+    """A cache row that overflowed fp16 in one key component: queries whose score there is -inf ignore it."""
+    P, t0 = 5, 90
+    Q, k, v = _inputs(P, t0)
+    Q.view(B, P, H, 64)[..., 7] = -0.5                    # exact in fp16: its lo half is 0
+    k[:, 1, 40, :, 7] = float('inf')
+    _check(_run(engine, kernel, Q, k, v, t0, P), Q, k, v, t0, P)
+    engine.check()

@@ -503,7 +503,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_embed_ln(const int* __restr
   const bool in = k8 < D;
   int x = tok[m];
   x = x < 0 ? 0 : (x >= V ? V - 1 : x);
-  int pos = *tp + m % P;
+  int pos = *tp + (P == 1 ? 0 : m % P);
   pos = pos < 0 ? 0 : (pos >= npos ? npos - 1 : pos);
   float v[8] = {}, wv[8] = {}, bv[8] = {};
   if (in) {
@@ -610,7 +610,7 @@ __device__ __forceinline__ void pf_epi8(int mode, int m, int n, float* v, const 
   unsigned short h[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) h[j] = f2h(v[j]);
-  const size_t at = ((size_t)(m / P * L + layer) * tmax + pos) * D + (n % D);
+  const size_t at = ((size_t)((P == 1 ? m : m / P) * L + layer) * tmax + pos) * D + (n % D);
   *(vh_u32x4*)((n < 2 * D ? kc : vc) + at) =
       vh_u32x4{h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16), h[4] | ((unsigned)h[5] << 16),
                h[6] | ((unsigned)h[7] << 16)};
@@ -650,7 +650,7 @@ __device__ __forceinline__ void pf_mgemm_body(
   if (eok) {
     if (bias && mode != 2) unpack8(ld16(bias + en), eb);
     if (mode == 1) pf_ld8f(out + (size_t)em * ldo + en, ez);
-    if (mode == 3) epos = *tp + em % P;
+    if (mode == 3) epos = *tp + (P == 1 ? 0 : em % P);
   }
   // weight fragments: nontemporal (WNT) where the model's weights cannot stay
   // in the memory-side cache between steps (the host picks the kernel)
@@ -898,119 +898,339 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_frag(const float* __
 }
 
 // ---------------------------------------------------------------- attention
-// One wave per (row m, head h): scores of the query against cache positions
-// 0 .. t0 + p (gpt2.vst Q5: dot over e, divided by 8; eight lanes per
-// position, each a 16-byte piece of the key row, the partial dots added
-// across them),
-// the max-subtracted softmax (Q6), and the weighted values (Q7: eight lanes
-// per position, 8 dims each), read from the fp16 cache the qkv product just
-// wrote. F receives the head's output, row m, in fragment order.
-// `ws` holds each wave's scores, then weights, for up to PF_TMAX positions.
-extern "C" __global__ __launch_bounds__(256) void pf_attn(const float* __restrict__ Q, const vh_half* __restrict__ kc,
-                                                           const vh_half* __restrict__ vc, int M, int P,
-                                                           const int* __restrict__ tp, int layer, int L, int tmax,
-                                                           int H, vh_half* __restrict__ F, int MT,
-                                                           unsigned* __restrict__ err) {
-  __shared__ float ws[VNWAVE][PF_TMAX];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int item = blockIdx.x * VNWAVE + wave;
-  const bool live = item < M * H;
-  const int m = live ? item / H : 0, h = live ? item % H : 0;
-  const int D = H * PF_E;
-  const int b = m / P, at = *tp + m % P;
-  const int pos = at < tmax ? at : tmax - 1;
-  const size_t base = (size_t)(b * L + layer) * tmax * D + (size_t)h * PF_E;
-  // scores: eight lanes per position (lane 8g + c holds dims 8c .. 8c + 7,
-  // one 16-byte load), positions g, g + 8, .. of the wave's 8 lane groups,
-  // four in flight per lane; the eight partial dots added across the group
+// Prefill attention on the matrix cores: a block of four waves makes 64 queries
+// of one (batch row, head), 16 to a wave, over the cache positions up to its
+// last query's in tiles of 64, with a running maximum, sum and weighted
+// values (gpt2.vst Q5-Q7: dot over e, divided by 8; max-subtracted softmax;
+// weighted values), read from the fp16 cache the qkv product just wrote.
+// Scores are K Q^T (K tile rows x 16 queries) and outputs V^T P^T (64 dims x
+// 16 queries), so that a lane holds values of one query (lane % 16) in both,
+// and the weights of a tile feed the second product from the registers the
+// first left them in: the instruction's fold position 8q + e of lane group q
+// stands for cache position 4q + e (e < 4) and 16 + 4q + e - 4 of a tile's 32,
+// and V is staged in that order. Queries (scaled by a power of two per query,
+// so that any fp32 magnitude splits) and softmax weights are split into fp16
+// halves like a product's activations (22 bits), each half in its own
+// accumulator. A score whose hi part is infinite is that infinity (the cache
+// may hold one, and 0 * inf of the lo part would make it a NaN).
+// What bounds it: vector work on the scores (exponentials, maxima, splits;
+// about 3 x the matrix-core time); few queries: the chain of tiles, 1.3 us
+// each. GPT-2 small, 32 x 768: 134 us a layer against 1198 with a wave per
+// (query row, head), which read every cache row once per query; 8 x 128 6.9
+// against 19.7; medium 3 x 333 after 100 positions 59 -> 22.
+// F receives the head's output, row m, in fragment order.
+// One query over at most 64 positions by one wave, in fp32 throughout: eight
+// lanes per position for the dots (the partial dots added across them), a
+// lane per position for the weights, eight lanes of 8 dims for each residue of
+// the positions mod 8 in the weighted values. `ws`: 64 floats of LDS.
+__device__ __forceinline__ void pf_attn_short(const float* __restrict__ qp, const vh_half* __restrict__ kb,
+                                              const vh_half* __restrict__ vb, int D, int pos, float* ws, int lane,
+                                              float* o) {
   const int g = lane >> 3, c8 = lane & 7;
   float qv[8];
-  {
-    const float* qp = Q + (size_t)m * D + h * PF_E + 8 * c8;
-    const vh_f32x4 q0 = live ? *(const vh_f32x4*)qp : vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const vh_f32x4 q1 = live ? *(const vh_f32x4*)(qp + 4) : vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    qv[0] = q0[0]; qv[1] = q0[1]; qv[2] = q0[2]; qv[3] = q0[3];
-    qv[4] = q1[0]; qv[5] = q1[1]; qv[6] = q1[2]; qv[7] = q1[3];
-  }
+  pf_ld8f(qp + 8 * c8, qv);
   float mx = -INFINITY;
-  if (live) {
-    for (int s0 = g; s0 <= pos; s0 += 8 * 4) {
-      vh_u32x4 kr[4];
+  for (int s = g; s <= pos; s += 8) {
+    float kv[8], acc = 0.0f;
+    unpack8(ld16(kb + (size_t)s * D + 8 * c8), kv);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int s = s0 + 8 * u;
-        kr[u] = s <= pos ? ld16(kc + base + (size_t)s * D + 8 * c8) : vh_u32x4{0u, 0u, 0u, 0u};
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        float kv[8];
-        unpack8(kr[u], kv);
-        float acc = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc = fmaf(qv[j], kv[j], acc);
-        acc += __shfl_xor(acc, 1, 64);
-        acc += __shfl_xor(acc, 2, 64);
-        acc += __shfl_xor(acc, 4, 64);
-        const int s = s0 + 8 * u;
-        if (s <= pos) {
-          const float sc = acc * 0.125f;      // / 8, exact
-          if (c8 == 0) ws[wave][s] = sc;
-          mx = fmaxf(mx, sc);
-        }
-      }
-    }
+    for (int j = 0; j < 8; ++j) acc = fmaf(qv[j], kv[j], acc);
+    acc += __shfl_xor(acc, 1, 64);
+    acc += __shfl_xor(acc, 2, 64);
+    acc += __shfl_xor(acc, 4, 64);
+    const float sc = acc * 0.125f;                                 // / 8, exact
+    if (c8 == 0) ws[s] = sc;
+    mx = fmaxf(mx, sc);
   }
   mx = wave_red_max(mx);
-  float sum = 0.0f;
-  if (live) {
-    for (int s = lane; s <= pos; s += 64) {
-      const float ex = expf(ws[wave][s] - mx);
-      ws[wave][s] = ex;
-      sum += ex;
-    }
+  const float ex = lane <= pos ? expf(ws[lane] - mx) : 0.0f;
+  const float sum = wave_red_sum(ex);
+  ws[lane] = ex / sum;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = 0.0f;
+  for (int s = g; s <= pos; s += 8) {
+    float v[8];
+    unpack8(ld16(vb + (size_t)s * D + 8 * c8), v);
+    const float w = ws[s];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = fmaf(w, v[j], o[j]);
   }
-  sum = wave_red_sum(sum);
-  if (live) {
-    for (int s = lane; s <= pos; s += 64) ws[wave][s] = ws[wave][s] / sum;
-  }
-  vh_lds_sync();
-  if (live) {
-    // lane 8a + b sums positions s = a (mod 8) over dims 8b..8b+7 (one 16-byte
-    // load of a row per position), four positions of its residue in flight;
-    // then the eight residues are added across lanes
-    const int a = lane >> 3, b = lane & 7;
-    float o[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s0 = 0; s0 <= pos; s0 += 32) {
-      vh_u32x4 vr[4];
-      float wv[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int s = s0 + 8 * u + a;
-        const bool in = s <= pos;
-        vr[u] = in ? ld16(vc + base + (size_t)s * D + 8 * b) : vh_u32x4{0u, 0u, 0u, 0u};
-        wv[u] = in ? ws[wave][s] : 0.0f;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        float v[8];
-        unpack8(vr[u], v);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = fmaf(wv[u], v[j], o[j]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      o[j] += __shfl_xor(o[j], 8, 64);
-      o[j] += __shfl_xor(o[j], 16, 64);
-      o[j] += __shfl_xor(o[j], 32, 64);
-    }
-    if (a == 0) {
-      bool bad = false;
-      pf_frag_put8(F, MT, D / 32, m, h * PF_E + 8 * b, o, bad);
-      if (bad) stc_u(err, VH_ERR_RANGE);
-    }
+  for (int j = 0; j < 8; ++j) {
+    o[j] += __shfl_xor(o[j], 8, 64);
+    o[j] += __shfl_xor(o[j], 16, 64);
+    o[j] += __shfl_xor(o[j], 32, 64);
   }
 }
+
+// With SPLIT a block makes 16 queries: its waves take every fourth tile of
+// positions each, staged for themselves, and combine at the end: where few
+// queries would leave waves or most of the chip idle over a long cache
+// (GPT-2 small, 3 tokens after 900 positions: 21.6 -> 10.8 us a launch). A
+// prompt of at most PF_SHORT tokens that sees at most 64 positions goes a
+// query at a time instead (pf_attn_short; no slower: one tile has no parts to
+// split).
+#define PF_SHORT 8
+template <bool SPLIT>
+__device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const vh_half* __restrict__ kc,
+                                             const vh_half* __restrict__ vc, int B, int P, const int* __restrict__ tp,
+                                             int layer, int L, int tmax, int H, vh_half* __restrict__ F, int MT,
+                                             unsigned* __restrict__ err) {
+  constexpr int QT = SPLIT ? 16 : 64, NB = SPLIT ? 4 : 2;          // queries of a block; staged tiles
+  constexpr int NK = SPLIT ? 8 : 2, NV = SPLIT ? 4 : 1;            // a lane's pieces of a staged tile
+  __shared__ __attribute__((aligned(16))) vh_u32x4 lk[NB][512];    // [position tile][k-step of dims][lane]
+  __shared__ __attribute__((aligned(16))) vh_u32x4 lv[NB][512];    // [dim tile][k-step of positions][lane]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int r = lane & 15, q = lane >> 4;
+  const int nq = (P + QT - 1) / QT, T = B * H * nq;
+  // contiguous runs of blocks per XCD (blockIdx % 8): a (row, head)'s blocks
+  // share its cache rows in one L2; within it the longest first
+  const int per = (T + 7) / 8, id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || id >= T) return;            // grid: 8 * ceil(T / 8) blocks
+  const int p0 = (nq - 1 - id % nq) * QT, h = id / nq % H, b = id / nq / H;
+  const int D = H * PF_E, t0 = *tp;
+  const size_t base = (size_t)(b * L + layer) * tmax * D + (size_t)h * PF_E;
+  const int w0 = SPLIT ? p0 : p0 + 16 * wave;                      // the wave's first query
+  const int pq = w0 + r;                                           // this lane's query
+  const bool live = pq < P;
+  const int lim = min(t0 + min(pq, P - 1), tmax - 1);              // its last position
+  const int last = min(t0 + min(p0 + QT, P) - 1, tmax - 1);     // the block's
+  const int wlast = min(t0 + min(w0 + 15, P - 1), tmax - 1);       // the wave's, and its first query's
+  const int wfirst = min(t0 + min(w0, P - 1), tmax - 1);
+  const bool wlive = w0 < P;
+  const int nt = last < 0 ? 0 : last / 64 + 1;
+  if (SPLIT && P <= PF_SHORT && last < 64) {
+    bool bad = false;
+    for (int p = wave; p < P; p += 4) {
+      float o[8];
+      pf_attn_short(Q + ((size_t)b * P + p) * D + h * PF_E, kc + base, vc + base, D, min(t0 + p, tmax - 1),
+                    (float*)lk[wave], lane, o);
+      if (lane < 8) pf_frag_put8(F, MT, D / 32, b * P + p, h * PF_E + 8 * lane, o, bad);
+    }
+    if (bad) stc_u(err, VH_ERR_RANGE);
+    return;
+  }
+  // the query, scaled to below 1 by 2^-e, in halves: dims 32 s + 8 q .. + 7
+  vh_u32x4 qh[2], ql[2];
+  float k2;                                                        // 2^e / 8 log2(e): scores in powers of 2
+  {
+    const float* qp = Q + ((size_t)b * P + min(pq, P - 1)) * D + h * PF_E + 8 * q;
+    float v[2][8];
+    float mx = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const vh_f32x4 a = *(const vh_f32x4*)(qp + 32 * s), c = *(const vh_f32x4*)(qp + 32 * s + 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[s][j] = a[j];
+        v[s][4 + j] = c[j];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mx = fmaxf(mx, __builtin_fabsf(v[s][j]));
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    int e = 0;
+    if (mx > 0.0f && mx < INFINITY) e = max(__builtin_amdgcn_frexp_expf(mx), -100);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[s][j] = __builtin_ldexpf(v[s][j], -e);
+      vh_split8s(v[s], qh[s], ql[s]);
+    }
+    k2 = __builtin_ldexpf(0.125f * 1.44269504088896341f, e);
+  }
+  // staging: keys as they are, row 16 i + r of the tile in 16-byte pieces
+  // c = 4 j + q; values of positions 4 va .. + 3, dims 4 vd .. + 3, transposed
+  // in registers. A tile is staged by the block, or with SPLIT by each wave.
+  // Positions past the last are read as the last (their weights are 0).
+  const int sl0 = SPLIT ? 0 : wave, vd = tid & 15;
+  vh_u32x4 kr[NK];
+  vh_u32x2 vr[NV][4];
+  auto gload = [&](int t) {
+#pragma unroll
+    for (int n = 0; n < NK; ++n) {
+      const int kp = min(64 * t + 16 * (sl0 + n / 2) + r, last);
+      kr[n] = ld16(kc + base + (size_t)kp * D + 8 * (4 * (n & 1) + q));
+    }
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int vp = min(64 * t + 4 * (4 * (sl0 + n) + q) + i, last);
+        vr[n][i] = ld8(vc + base + (size_t)vp * D + 4 * vd);
+      }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int n = 0; n < NK; ++n) lk[buf][(2 * (sl0 + n / 2) + (n & 1)) * 64 + lane] = kr[n];
+    // dims 4 vd + j: dim tile vd / 4, row 4 (vd % 4) + j of it; positions
+    // 4 va ..: k-step va / 8, half (va % 8) / 4 of lane group va % 4's eight
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int va = 4 * (sl0 + n) + q;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const unsigned sel = j & 1 ? 0x07060302u : 0x05040100u;
+        const vh_u32x2 w = {__builtin_amdgcn_perm(vr[n][1][j >> 1], vr[n][0][j >> 1], sel),
+                            __builtin_amdgcn_perm(vr[n][3][j >> 1], vr[n][2][j >> 1], sel)};
+        const int piece = (vd / 4 * 2 + va / 8) * 64 + (va & 3) * 16 + 4 * (vd & 3) + j;
+        *((vh_u32x2*)&lv[buf][piece] + ((va & 7) >> 2)) = w;
+      }
+    }
+  };
+  vh_f32x4 oh[4], ol[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) oh[d] = ol[d] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float m2 = -INFINITY, sum = 0.0f;      // largest score in powers of 2; the sum of this lane's positions
+  if constexpr (SPLIT) {
+    if (wave < nt) gload(wave);
+  } else if (nt > 0) {
+    gload(0);
+    put(0);
+    if (nt > 1) gload(1);
+  }
+  for (int t = SPLIT ? wave : 0; t < nt; t += SPLIT ? 4 : 1) {
+    if constexpr (SPLIT) {
+      put(wave);                           // the wave's own tile: its LDS operations are in order
+      if (t + 4 < nt) gload(t + 4);
+    } else {
+      vh_lds_sync();
+      if (t + 1 < nt) {                    // the other buffer: read before the previous barrier
+        put((t + 1) & 1);
+        if (t + 2 < nt) gload(t + 2);
+      }
+      if (!wlive || 64 * t > wlast) continue;
+    }
+    const int buf = SPLIT ? wave : t & 1;
+    const vh_u32x4 *K = lk[buf], *V = lv[buf];
+    float s[4][4], big = 0.0f;
+    vh_f32x4 sh[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      vh_f32x4 sl = {0.0f, 0.0f, 0.0f, 0.0f};
+      sh[i] = sl;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const vh_u32x4 kf = K[(2 * i + k) * 64 + lane];
+        sh[i] = vh_mfma(kf, qh[k], sh[i]);
+        sl = vh_mfma(kf, ql[k], sl);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s[i][j] = vh_hilo(sh[i][j], sl[j]);
+        big = fmaxf(big, __builtin_fabsf(sh[i][j]));
+      }
+    }
+    if (__any(big == INFINITY)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[i][j] = __builtin_isinf(sh[i][j]) ? sh[i][j] : s[i][j];
+    }
+    if (64 * t + 63 > wfirst) {                                    // a tile that some query sees in part
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[i][j] = 64 * t + 16 * i + 4 * q + j <= lim ? s[i][j] : -INFINITY;
+    }
+    float bm = s[0][0];
+#pragma unroll
+    for (int n = 1; n < 16; ++n) bm = fmaxf(bm, s[n >> 2][n & 3]);
+    bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
+    bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+    const float n2 = fmaxf(m2, bm * k2);
+    const float ref = n2 == -INFINITY ? 0.0f : n2;                 // no score above -inf yet: all weights 0
+    if (__any(n2 != m2)) {
+      const float c = __builtin_amdgcn_exp2f(m2 - ref);            // 0 while m2 is -inf
+      sum *= c;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          oh[d][j] *= c;
+          ol[d][j] *= c;
+        }
+      m2 = n2;
+    }
+    vh_u32x4 ph[2], pl[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      vh_h8 hi, lo;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float w = __builtin_amdgcn_exp2f(fmaf(s[2 * k + (j >> 2)][j & 3], k2, -ref));
+        sum += w;
+        hi[j] = (_Float16)w;
+        lo[j] = (_Float16)fmaf((float)hi[j], -VH_LO_SCALE, w * VH_LO_SCALE);     // (w - hi) 2^11, exact
+      }
+      ph[k] = __builtin_bit_cast(vh_u32x4, hi);
+      pl[k] = __builtin_bit_cast(vh_u32x4, lo);
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const vh_u32x4 vf = V[(2 * d + k) * 64 + lane];
+        oh[d] = vh_mfma(vf, ph[k], oh[d]);
+        ol[d] = vh_mfma(vf, pl[k], ol[d]);
+      }
+  }
+  sum += __shfl_xor(sum, 16, 64);
+  sum += __shfl_xor(sum, 32, 64);
+  float o[4][4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[d][j] = vh_hilo(oh[d][j], ol[d][j]);
+  if constexpr (SPLIT) {
+    // each wave's maximum, sum and output rescaled to the common maximum and
+    // added in wave order; wave w then writes dim tile w
+    float *om = (float*)lk[0], *ow = (float*)lv[0];                // [wave][maximum, sum][16], [wave][dim tile][j][lane]
+    __syncthreads();
+    if (q == 0) {
+      om[wave * 32 + r] = m2;
+      om[wave * 32 + 16 + r] = sum;
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ow[((wave * 4 + d) * 4 + j) * 64 + lane] = o[d][j];
+    __syncthreads();
+    float m = om[r];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) m = fmaxf(m, om[w * 32 + r]);
+    sum = 0.0f;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float wm = om[w * 32 + r], f = wm == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(wm - m);   // no score: 0
+      sum = fmaf(om[w * 32 + 16 + r], f, sum);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = fmaf(ow[((w * 4 + wave) * 4 + j) * 64 + lane], f, v[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[0][j] = v[j];
+  }
+  if (!live) return;
+  bool bad = false;
+#pragma unroll
+  for (int d = 0; d < (SPLIT ? 1 : 4); ++d) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[d][j] = lim < 0 ? 0.0f : o[d][j] / sum;
+    pf_frag_put4(F, MT, D / 32, b * P + pq, h * PF_E + 16 * (SPLIT ? wave : d) + 4 * q, o[d], bad);
+  }
+  if (bad) stc_u(err, VH_ERR_RANGE);
+}
+#define PF_ATTN(name, split)                                                                                        \
+  extern "C" __global__ __launch_bounds__(256, 2) void name(                                                        \
+      const float* __restrict__ Q, const vh_half* __restrict__ kc, const vh_half* __restrict__ vc, int B, int P,    \
+      const int* __restrict__ tp, int layer, int L, int tmax, int H, vh_half* __restrict__ F, int MT,               \
+      unsigned* __restrict__ err) {                                                                                 \
+    pf_attn_body<split>(Q, kc, vc, B, P, tp, layer, L, tmax, H, F, MT, err);                                        \
+  }
+PF_ATTN(pf_attn, false)
+PF_ATTN(pf_attn16, true)
 
 // One position per row (a decode step): one block per (row m, head h), every
 // thread of the block on the positions 0 .. t0, so that a step's cache rows

@@ -34,8 +34,8 @@ PRELUDE_SRC = Path(__file__).resolve().parent / 'hip' / 'prelude.h'
 BLOCK = 256
 CHUNK = 64                    # products' fold lengths are multiples of this (two 32-deep k-steps)
 HEAD = 64
-KERNELS = ('pf_ln', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn1', 'pf_argmax_part', 'pf_argmax', 'pf_mgemm1',
-           'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n', 'pf_mgemm2n', 'pf_mgemm4n', 'pf_reduce_frag', 'pf_attn1s',
+KERNELS = ('pf_ln', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn16', 'pf_attn1', 'pf_argmax_part', 'pf_argmax',
+           'pf_mgemm1', 'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n', 'pf_mgemm2n', 'pf_mgemm4n', 'pf_reduce_frag', 'pf_attn1s',
            'pf_mhead1', 'pf_mhead2', 'pf_mhead4', 'pf_embed_ln', 'pf_pgemm128', 'pf_pgemm64',
            'pf_pgemm64w', 'pf_pgemm32')
 ARGMAX_SPLIT = 32             # blocks per row of the output-head argmax (same box, 16 -> 32: GPT-2 small 32 rows
@@ -55,6 +55,11 @@ MEM_CACHE_BYTES = 256 << 20   # the device's memory-side cache: decode products 
                               # larger load them nontemporal (same box: XL B=64 3.000 -> 2.944 ms per step,
                               # medium B=16 0.958 -> 0.916; GPT-2 small's 247 MB stay in that cache between
                               # steps, nontemporal there: 32 rows 0.548 -> 0.553)
+ORDERED_TOKENS, ORDERED_LAYERS = 8, 24      # see ordered()
+ATTN_SPLIT_BLOCKS = 512       # prefill attention with at most this many blocks of 16 queries (two per CU, all
+                              # resident) splits each one's positions over its waves (pf_attn16). us a launch, pf_attn
+                              # / pf_attn16, GPT-2 small: 1 x 200 after 700 positions (156 such blocks) 22.0 / 10.6,
+                              # 20 x 32 after 365 (480) 13.3 / 11.7, 60 x 3 (720) 6.3 / 8.2, 8 x 128 (768) 6.9 / 10.3
 ATTN_ONE_PASS_BLOCKS = 1024   # decode passes with at most this many (row, head) blocks read each cache row in
                               # one pass (pf_attn1s), more in two (pf_attn1: keys, then values; fewer
                               # registers, more blocks resident). Same box, two -> one pass: small 16 / 24 rows
@@ -104,6 +109,31 @@ def pgemm_plan(M, N, K, split):
     (``split``: whether its fold may be split): the least ``pgemm_us``."""
     return min(((name, ks) for name in PG_TILES for ks in ((1, 2, 3, 4, 6) if split else (1,)) if K // 64 >= 2 * ks
                 or ks == 1), key=lambda c: pgemm_us(c[0], M, N, K, c[1]))
+
+
+def ordered(P, L):
+    """Whether a prompt of P tokens in a model of L layers goes through the
+    products and the attention whose order of sums is fixed by the model alone
+    (``ordered_parts``, ``pf_attn_short``). From an empty cache a short
+    prompt's attention averages over few positions, so a new cache row that
+    lies next to an fp16 rounding boundary and goes the other way is carried
+    on almost undiminished, layer after layer: with another order of sums,
+    XL's cache rows come out 1.9e-4 .. 2.8e-4 apart (2-norm) at 3-6 tokens,
+    2.1e-4 at 8, 1.6e-4 at 16; medium's 1.6e-4 .. 2.3e-4 at 3-4; GPT-2 small's
+    below 1.5e-4."""
+    return 1 < P <= ORDERED_TOKENS and L >= ORDERED_LAYERS
+
+
+def ordered_parts(M, N, K):
+    """Fold parts of an ordered product: about 384 output tiles of 64 x 64
+    times parts, each part at least 256 deep."""
+    return max(1, min(-(-384 // (-(-M // 64) * -(-N // 64))), K // 256))
+
+
+def prefill_attn(B, P, H, ordered=False):
+    """Kernel and blocks of the prefill attention of B rows of P positions."""
+    few = B * H * -(-P // 16)
+    return ('pf_attn16', few) if ordered or few <= ATTN_SPLIT_BLOCKS else ('pf_attn', B * H * -(-P // 64))
 
 
 def frag_weights(Wt):
@@ -270,29 +300,18 @@ class Prefill:
         self._launch(f'pf_mgemm{mt}' + ('n' if self._weights_nt() else ''), nb * ks,
                      [_p(Af), _p(Wf), _i(KT), _i(NT), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out), _i(ldo)]
                      + t_args + [_p(ws), _p(F), _p(self.err)], block=MG_WAVES * 64)
-        if ks == 1:
-            return False
-        if mode == MODE_RESID and ln is not None:
-            w, b, Fo = ln
-            self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _p(w), _p(b), _p(Fo),
-                                             _i(mt), _p(self.err)])
-            return True
-        if mode == MODE_GELU:
-            self._launch('pf_reduce_frag', -(-M * (N // 8) // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(F),
-                                                                       _i(mt), _p(self.err)])
-        else:
-            self._launch('pf_reduce', -(-M * N // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out),
-                                                            _i(ldo)] + t_args)
-        return False
+        return self._reduce(ws, ks, bias, M, N, mt, mode, out, ldo, P, layer, F, ln)
 
-    def _pgemm(self, Af, K, wname, layer, N, mode, bias=None, out=None, ldo=0, F=None, ln=None, M=1, P=1):
-        """One product of any number of rows (``pf_pgemm*``), as ``_mgemm``;
-        only a residual product with a LayerNorm after it splits its fold
-        (its reduction adds no launch)."""
+    def _pgemm(self, Af, K, wname, layer, N, mode, bias=None, out=None, ldo=0, F=None, ln=None, M=1, P=1, ks=None):
+        """One product of any number of rows (``pf_pgemm*``), as ``_mgemm``.
+        With ``ks`` None only a residual product with a LayerNorm after it
+        splits its fold (its reduction adds no launch); else in ``ks`` parts."""
         m = self.m
         KT, NT, MT = K // 32, -(-N // 16), _mtiles(M)
-        split = mode == MODE_RESID and ln is not None and ldo == N
-        name, ks = pgemm_plan(M, N, K, split)
+        if ks is None:
+            name, ks = pgemm_plan(M, N, K, mode == MODE_RESID and ln is not None and ldo == N)
+        else:
+            name = 'pf_pgemm32'
         ws = self._workspace(ks * M * N) if ks > 1 else None
         Wf = self._frag(wname)
         Wf = Wf[layer] if layer is not None else Wf
@@ -313,15 +332,34 @@ class Prefill:
                      [_p(Af), _p(Wf), _i(MT), _i(KT), _i(NT), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out),
                       _i(ldo), _p(m.keys), _p(m.vals), _i(P), _p(m.t), _i(layer or 0), _i(m.L), _i(m.tmax), _p(ws),
                       _p(F), _p(self.err)], block=waves * 64)
-        if ks > 1:
+        return self._reduce(ws, ks, bias, M, N, MT, mode, out, ldo, P, layer, F, ln)
+
+    def _reduce(self, ws, ks, bias, M, N, MT, mode, out, ldo, P, layer, F, ln):
+        """The launch that adds a split product's parts, if there are any;
+        returns whether it made the LayerNorm ``ln`` too."""
+        m = self.m
+        if ks == 1:
+            return False
+        if mode == MODE_RESID and ln is not None:
             w, b, Fo = ln
             self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _p(w), _p(b), _p(Fo),
                                              _i(MT), _p(self.err)])
-        return ks > 1
+            return True
+        if mode == MODE_GELU:
+            self._launch('pf_reduce_frag', -(-M * (N // 8) // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(F),
+                                                                       _i(MT), _p(self.err)])
+        else:
+            self._launch('pf_reduce', -(-M * N // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out),
+                                                            _i(ldo), _p(m.keys), _p(m.vals), _i(P), _p(m.t),
+                                                            _i(layer or 0), _i(m.L), _i(m.tmax)])
+        return False
 
-    def _product(self, *a, M, **kw):
+    def _product(self, Af, K, wname, layer, N, mode, M, ordered=False, **kw):
         """A product on the kernels for its row count (True: the LayerNorm
         that follows it is done)."""
+        a = (Af, K, wname, layer, N, mode)
+        if ordered:
+            return self._pgemm(*a, M=M, ks=ordered_parts(M, N, K), **kw)
         return (self._mgemm if M <= FEW_ROWS else self._pgemm)(*a, M=M, **kw)
 
     def _weights_nt(self):
@@ -439,6 +477,7 @@ class Prefill:
         W = m.W
         Z, Q, AF, GF, err = buf['Z'], buf['Q'], buf['AF'], buf['GF'], self.err
         mt = _mtiles(M)
+        fixed = ordered(P, L)
 
         def norm(w, b, to, rows, row0=0, stride=1):
             self._launch('pf_ln', rows, [_p(Z), _i(row0), _i(stride), _p(w), _p(b), _i(D), _p(to), _i(_mtiles(rows)),
@@ -449,24 +488,25 @@ class Prefill:
         for layer in range(L):
             def lw(name, layer=layer):
                 return W[name][layer]
-            self._product(AF, D, 'qkvw', layer, 3 * D, MODE_QKV, bias=lw('qkvb'), out=Q, ldo=D, M=M, P=P)
+            self._product(AF, D, 'qkvw', layer, 3 * D, MODE_QKV, bias=lw('qkvb'), out=Q, ldo=D, M=M, P=P,
+                          ordered=fixed)
             cache = [_p(Q), _p(m.keys), _p(m.vals)]
             if P == 1:          # a block per (row, head) (GPT-2 small, 32 rows, 1024 positions:
                                 # 1.32 -> 1.07 ms per step against a wave per (row, head))
                 self._launch(self._attn1(), B * H, cache + [_p(m.t), _i(layer), _i(L), _i(m.tmax), _i(H), _p(AF),
                                                             _i(mt), _p(err)])
             else:
-                self._launch('pf_attn', -(-M * H // (BLOCK // 64)),
-                             cache + [_i(M), _i(P), _p(m.t), _i(layer), _i(L), _i(m.tmax), _i(H), _p(AF), _i(mt),
-                                      _p(err)])
+                name, blocks = prefill_attn(B, P, H, fixed)
+                self._launch(name, 8 * -(-blocks // 8), cache + [_i(B), _i(P), _p(m.t), _i(layer), _i(L), _i(m.tmax),
+                                                                 _i(H), _p(AF), _i(mt), _p(err)])
             if not self._product(AF, D, 'ow', layer, D, MODE_RESID, bias=lw('ob'), out=Z, ldo=D,
-                                 ln=(lw('ln2w'), lw('ln2b'), AF), M=M):
+                                 ln=(lw('ln2w'), lw('ln2b'), AF), M=M, ordered=fixed):
                 norm(lw('ln2w'), lw('ln2b'), AF, M)
-            self._product(AF, D, 'fcw', layer, F, MODE_GELU, bias=lw('fcb'), F=GF, M=M)
+            self._product(AF, D, 'fcw', layer, F, MODE_GELU, bias=lw('fcb'), F=GF, M=M, ordered=fixed)
             last = layer + 1 == L
             nxt = (W['lnfw'], W['lnfb'], AF) if last else (lw('ln1w', layer + 1), lw('ln1b', layer + 1), AF)
             normed = self._product(GF, F, 'pw', layer, D, MODE_RESID, bias=lw('pb'), out=Z, ldo=D,
-                                   ln=nxt if P == 1 or not last else None, M=M)
+                                   ln=nxt if P == 1 or not last else None, M=M, ordered=fixed)
             if not normed and not (last and P > 1):
                 norm(*nxt, M)
         if P > 1:               # the final norm: each row's last position
