@@ -142,3 +142,29 @@ def test_more_than_64_rows_decode_and_prefill_like_fewer():
         m.check()
         got.append(torch.stack(lg).cpu().numpy())
     assert np.abs(got[0] - got[1]).max() < 1e-3
+
+
+@pytest.mark.parametrize('D', [64, 1024, 1088, 2048])
+@pytest.mark.parametrize('M', [1, 17, 48])
+def test_layer_norm_of_sixteen_rows_a_block_matches_64_bits(engine, D, M):
+    """pf_lnm*: widths at the ends of each kernel's range, rows around a block's 16."""
+    import torch
+    from vesta import prefill as pf
+    e = engine._pf
+    gen = torch.Generator(device='cuda').manual_seed(D + M)
+    X, w, b = (torch.randn(*s, generator=gen, device='cuda') for s in ((M, D), (D,), (D,)))
+    w, b = w.half(), b.half()
+    F = torch.zeros(2 * 16 * pf._mtiles(M) * D, dtype=torch.float16, device='cuda')
+    e._plan = []
+    p, i = pf._p, pf._i
+    e._launch('pf_lnm8' if D <= 1024 else 'pf_lnm16', -(-M // 16), [p(X), i(M), i(D), p(w), p(b), p(F),
+                                                                     i(pf._mtiles(M)), p(e.err)])
+    plan, e._plan = e._plan, []
+    e._replay(plan)
+    x = X.double()
+    c = x - x.mean(-1, keepdim=True)
+    y = c / torch.sqrt((c * c).mean(-1, keepdim=True) + 1e-5)
+    want = y * w.double() + b.double()
+    # sums of D fp32 terms (2^-24 each, at most sqrt(D) long along a lane, lanes and waves), four roundings, 22 bits
+    _close(_unfrag(F, M, D), want, (2.0 ** -21 + D ** 0.5 * 2.0 ** -24) * ((y * w.double()).abs() + b.double().abs() + 1))
+    e.check()

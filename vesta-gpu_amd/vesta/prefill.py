@@ -34,7 +34,7 @@ PRELUDE_SRC = Path(__file__).resolve().parent / 'hip' / 'prelude.h'
 BLOCK = 256
 CHUNK = 64                    # products' fold lengths are multiples of this (two 32-deep k-steps)
 HEAD = 64
-KERNELS = ('pf_ln', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn16', 'pf_attn1', 'pf_argmax_part', 'pf_argmax',
+KERNELS = ('pf_ln', 'pf_lnm8', 'pf_lnm16', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn16', 'pf_attn1', 'pf_argmax_part', 'pf_argmax',
            'pf_mgemm1', 'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n', 'pf_mgemm2n', 'pf_mgemm4n', 'pf_reduce_frag', 'pf_attn1s',
            'pf_mhead1', 'pf_mhead2', 'pf_mhead4', 'pf_embed_ln', 'pf_pgemm128', 'pf_pgemm64',
            'pf_pgemm64w', 'pf_pgemm32')
@@ -55,6 +55,9 @@ MEM_CACHE_BYTES = 256 << 20   # the device's memory-side cache: decode products 
                               # larger load them nontemporal (same box: XL B=64 3.000 -> 2.944 ms per step,
                               # medium B=16 0.958 -> 0.916; GPT-2 small's 247 MB stay in that cache between
                               # steps, nontemporal there: 32 rows 0.548 -> 0.553)
+LNM_ROWS = 1536               # LayerNorms of at least this many rows take a block per 16 rows (pf_lnm*; us a
+                              # launch, block per row / per 16 rows: 999 x 768 6.4 / 7.0, 2048 x 768 8.9 / 7.5, 999 x
+                              # 1600 8.7 / 12.1, 2048 x 1600 13.5 / 13.9, 4096 x 1600 24.6 / 16.0)
 ORDERED_TOKENS, ORDERED_LAYERS = 8, 24      # see ordered()
 ATTN_SPLIT_BLOCKS = 512       # prefill attention with at most this many blocks of 16 queries (two per CU, all
                               # resident) splits each one's positions over its waves (pf_attn16). us a launch, pf_attn
@@ -480,6 +483,10 @@ class Prefill:
         fixed = ordered(P, L)
 
         def norm(w, b, to, rows, row0=0, stride=1):
+            if rows >= LNM_ROWS and stride == 1:
+                self._launch('pf_lnm8' if D <= 1024 else 'pf_lnm16', -(-rows // 16),
+                             [_p(Z), _i(rows), _i(D), _p(w), _p(b), _p(to), _i(_mtiles(rows)), _p(err)])
+                return
             self._launch('pf_ln', rows, [_p(Z), _i(row0), _i(stride), _p(w), _p(b), _i(D), _p(to), _i(_mtiles(rows)),
                                          _p(err)])
         self._launch('pf_embed_ln', M, [_p(tok), _i(P), _p(m.t), _p(W['wte']), _p(W['wpe']), _p(Z), _i(D), _i(V),
