@@ -168,3 +168,26 @@ def test_layer_norm_of_sixteen_rows_a_block_matches_64_bits(engine, D, M):
     # sums of D fp32 terms (2^-24 each, at most sqrt(D) long along a lane, lanes and waves), four roundings, 22 bits
     _close(_unfrag(F, M, D), want, (2.0 ** -21 + D ** 0.5 * 2.0 ** -24) * ((y * w.double()).abs() + b.double().abs() + 1))
     e.check()
+
+
+@pytest.mark.parametrize('shape', [(2, 192, 3, 768), (1, 1600, 25, 6400)])
+def test_up_to_eight_rows_compute_what_more_rows_compute(shape):
+    """Products of at most 8 rows hold both halves of the activations in one operand tile; each row's sums are those of
+    the same rows in a batch of 9, bit for bit (the wider shape: waves with more k-steps than one batch of loads)."""
+    import torch
+    from vesta.gpt2 import VestaGPT2
+    from vesta.weights import GPT2Shape, RandomGPT2, random_prompts
+    hf = RandomGPT2(GPT2Shape(*shape, vocab=203), 6)
+    pr = torch.from_numpy(random_prompts(9, 4, 203, seed=4)).to('cuda', torch.int32)
+    got = []
+    for rows in (9, 8, 3, 1):
+        m = VestaGPT2(hf, batch=rows, tmax=16, engine='layered')
+        m.reset()
+        for k in range(4):
+            m.x.copy_(pr[:rows, k])
+            m.step()
+        m.check()
+        got.append((m.logits().clone(), m.keys.clone(), m.vals.clone()))
+    for rows, g in zip((8, 3, 1), got[1:]):
+        for a, b in zip(g, got[0]):
+            assert torch.equal(a, b[:rows])

@@ -755,7 +755,35 @@ __device__ __forceinline__ void pf_mgemm_body(
         acl[t][mt] = vh_mfma(a[1][mt], w[t], acl[t][mt]);
       }
   };
-  if (k1 - k0 <= PF_WFIRST) {
+  // up to 8 rows: the hi halves of rows 0-7 and the lo halves in one operand
+  // tile (its rows 0-7 and 8-15), so one product and one activation fragment a
+  // k-step; all of a wave's loads are issued at once, the activations (from L2)
+  // before the weights, which the products then wait for one by one (XL at one
+  // row: 7.9 -> 6.9 us a product, 2.08 -> 1.90 ms per step)
+  const bool packed = MT == 1 && M <= 8;
+  if (packed) {
+    const vh_u32x4* Ap = Af + ((lane & 8) ? plane : 0) + (lane & 0x37);
+    for (int kb8 = k0; kb8 < k1; kb8 += PF_WFIRST) {
+      vh_u32x4 a8[PF_WFIRST], w8[PF_WFIRST][MN];
+#pragma unroll
+      for (int j = 0; j < PF_WFIRST; ++j) a8[j] = kb8 + j < k1 ? Ap[(size_t)(kb8 + j) * 64] : vh_u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < PF_WFIRST; ++j)
+#pragma unroll
+        for (int t = 0; t < MN; ++t)
+          w8[j][t] = kb8 + j < k1 && nt0 + t < NT ? wld(((size_t)(nt0 + t) * KT + kb8 + j) * 64 + lane)
+                                                  : vh_u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < PF_WFIRST; ++j)
+        if (kb8 + j < k1)
+#pragma unroll
+          for (int t = 0; t < MN; ++t) acc[t][0] = vh_mfma(a8[j], w8[j][t], acc[t][0]);
+    }
+#pragma unroll
+    for (int t = 0; t < MN; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acl[t][0][v] = __shfl_xor(acc[t][0][v], 32, 64);     // rows 8 .. 15: the lo sums
+  } else if (k1 - k0 <= PF_WFIRST) {
     // all of the wave's weight fragments first (so they are in flight at once),
     // then the activation fragments one k-step ahead
     vh_u32x4 wall[PF_WFIRST][MN];
