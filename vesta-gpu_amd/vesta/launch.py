@@ -502,6 +502,14 @@ class Kernel:
                                  ctypes.c_void_p(stream)), 'static scratch read')
         return int(word.item())
 
+    def error_word_view(self):
+        """The error word ``check()`` reads, as a one-element view of ``bar`` (no
+        synchronisation), or None where it is elsewhere (the static scratch)."""
+        from .lower import BAR_ERROR
+        if getattr(self, '_noalloc_bar', None) is not None or self.bar.numel() <= BAR_ERROR:
+            return None
+        return self.bar[BAR_ERROR:BAR_ERROR + 1]
+
     def _noalloc_word(self):
         w = getattr(self, '_noalloc_word_t', None)
         if w is None:
