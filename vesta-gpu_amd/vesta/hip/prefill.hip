@@ -117,10 +117,11 @@ __device__ __forceinline__ void pf_epi(int mode, int m, int n, float c, const vh
 // global load one contiguous kilobyte and every LDS access conflict-free
 // without padding, and the halves are made once, by the activation's producer.
 // What bounds them: the matrix cores twice per product (hi and lo) at the
-// clock that load leaves; at 24576 x 2304 x 768 the 128 x 256 tile takes 192
-// us (453 TFLOP/s of the product, 906 of the matrix cores; hipBLASLt's fp16
+// clock that load leaves; at 24576 x 2304 x 768 the 128 x 256 tile takes 174
+// us (500 TFLOP/s of the product, 1000 of the matrix cores; hipBLASLt's fp16
 // product of the same operation count 171 us), where 64 x 64 tiles that
-// converted fp32 activations in every block took 380.
+// converted fp32 activations in every block took 380. With few tiles a CU it
+// is the tile's fixed part (first loads, epilogue: 4-8 us).
 // `ks` > 1 splits the fold over blocks: part p of tile t stores its sums in
 // ws[p][m][n] for pf_reduce_ln.
 //
@@ -144,62 +145,123 @@ __device__ __forceinline__ bool pf_tile(PfTile& tl, int MT, int NT, int ks) {
 }
 
 // A wave's TM x TN output tiles (from row tile mt0, column tile nt0) through
-// the epilogue of `mode`, or into ws[part] with a split fold.
+// the epilogue of `mode`, or into ws[part] with a split fold. Lane 16 q + r
+// holds row r, columns 4 q .. + 3 of each tile. All operands of a row of tiles
+// are loaded before any is used, and what differs by tile alone is scalar:
+// with a load, a wait and per-lane divisions for each tile the epilogue of the
+// 128 x 256 tile took about 8 us, a third of a 768-deep product (24576 x 2304
+// x 768 192 -> 174 us, 8192 x 4800 x 1600 237 -> 229).
 template <int TM, int TN>
 __device__ __forceinline__ void pf_pgemm_out(
     const vh_f32x4 (&ah)[TM][TN], const vh_f32x4 (&al)[TM][TN], int mt0, int nt0, int part, int ks, int MT,
     const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,
     vh_half* __restrict__ kc, vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer, int L, int tmax,
     float* __restrict__ ws, vh_half* __restrict__ F, unsigned* __restrict__ err) {
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 15, q4 = 4 * (lane >> 4), t0 = mode == 3 ? *tp : 0;
-  bool bad = false;
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int m0 = 16 * mt0 + r, n0 = 16 * nt0 + 4 * q;              // this lane's row of row tile 0, column of column tile 0
+  auto value = [&](int a, int b) {
+    return vh_f32x4{vh_hilo(ah[a][b][0], al[a][b][0]), vh_hilo(ah[a][b][1], al[a][b][1]),
+                    vh_hilo(ah[a][b][2], al[a][b][2]), vh_hilo(ah[a][b][3], al[a][b][3])};
+  };
+  if (ks > 1) {
+    float* w = ws + ((size_t)part * M + m0) * N + n0;
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+      if (m0 + 16 * a >= M) continue;
+#pragma unroll
+      for (int b = 0; b < TN; ++b)
+        if (n0 + 16 * b < N) *(vh_f32x4*)(w + (size_t)(16 * a) * N + 16 * b) = value(a, b);
+    }
+    return;
+  }
+  if (mode == 0) {                                                 // N of any size (the output head)
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+      for (int b = 0; b < TN; ++b) {
+        const vh_f32x4 v = value(a, b);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int m = m0 + 16 * a, n = n0 + 16 * b + j;
+          if (m < M && n < N) out[(size_t)m * ldo + n] = bias ? v[j] + h2f(bias[n]) : v[j];
+        }
+      }
+    return;
+  }
+  float bn[TN][4];
+#pragma unroll
+  for (int b = 0; b < TN; ++b) unpack4(ld8(bias + min(n0 + 16 * b, N - 4)), bn[b]);
+  if (mode == 1) {
+    float* o = out + (size_t)m0 * ldo + n0;
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+      if (m0 + 16 * a >= M) continue;
+      vh_f32x4 z[TN];
+#pragma unroll
+      for (int b = 0; b < TN; ++b)
+        z[b] = n0 + 16 * b < N ? *(const vh_f32x4*)(o + (size_t)(16 * a) * ldo + 16 * b) : vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int b = 0; b < TN; ++b) {
+        const vh_f32x4 v = value(a, b);
+        if (n0 + 16 * b < N)
+          *(vh_f32x4*)(o + (size_t)(16 * a) * ldo + 16 * b) =
+              vh_f32x4{(z[b][0] + v[0]) + bn[b][0], (z[b][1] + v[1]) + bn[b][1], (z[b][2] + v[2]) + bn[b][2],
+                       (z[b][3] + v[3]) + bn[b][3]};
+      }
+    }
+    return;
+  }
+  if (mode == 2) {
+    // fragment order: the lane's eight bytes of tile (mt0 + a, nt0 + b) are at a place of its own in half a fragment
+    bool bad = false;
+    const size_t at = (((q >> 1) * 16 + r) * 8) + (q & 1) * 4, plane = (size_t)MT * (N / 32) * 512;
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+      if (m0 + 16 * a >= M) continue;
+#pragma unroll
+      for (int b = 0; b < TN; ++b) {
+        if (n0 + 16 * b >= N) continue;
+        const vh_f32x4 v = value(a, b);
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        h4 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float g = pf_gelu(v[j] + bn[b][j]);
+          bad |= !(__builtin_fabsf(g) <= VH_HALF_MAX);
+          hi[j] = (_Float16)g;
+          lo[j] = (_Float16)((g - (float)hi[j]) * VH_LO_SCALE);
+        }
+        vh_half* f = F + ((size_t)(mt0 + a) * (N / 32) + ((nt0 + b) >> 1)) * 512 + ((nt0 + b) & 1) * 256 + at;
+        *(vh_u32x2*)f = __builtin_bit_cast(vh_u32x2, hi);
+        *(vh_u32x2*)(f + plane) = __builtin_bit_cast(vh_u32x2, lo);
+      }
+    }
+    if (bad) stc_u(err, VH_ERR_RANGE);
+    return;
+  }
+  // qkv: a 16-column tile is all queries, keys or values (D is a multiple of 64)
+  const int D = N / 3, t0 = *tp;
 #pragma unroll
   for (int a = 0; a < TM; ++a) {
-    const int m = 16 * (mt0 + a) + r;
+    const int m = m0 + 16 * a, bi = m / P, pos = t0 + m - bi * P;
     if (m >= M) continue;
+    const bool cached = pos >= 0 && pos < tmax;
+    const size_t row = ((size_t)(bi * L + layer) * tmax + pos) * D + 4 * q;
 #pragma unroll
     for (int b = 0; b < TN; ++b) {
-      const int n = 16 * (nt0 + b) + q4;
-      if (n >= N) continue;
-      float v[4];
+      const int nt = 16 * (nt0 + b);                               // uniform
+      if (nt >= N) continue;
+      vh_f32x4 v = value(a, b);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = vh_hilo(ah[a][b][j], al[a][b][j]);
-      if (ks > 1) {
-        *(vh_f32x4*)(ws + ((size_t)part * M + m) * N + n) = vh_f32x4{v[0], v[1], v[2], v[3]};
-        continue;
-      }
-      if (mode == 0) {                                  // N of any size (the output head)
-        for (int j = 0; j < 4; ++j)
-          if (n + j < N) out[(size_t)m * ldo + n + j] = bias ? v[j] + h2f(bias[n + j]) : v[j];
-        continue;
-      }
-      float bn[4];
-      unpack4(ld8(bias + n), bn);
-      if (mode == 1) {
-        float* o = out + (size_t)m * ldo + n;
-        const vh_f32x4 z = *(const vh_f32x4*)o;
-        *(vh_f32x4*)o = vh_f32x4{(z[0] + v[0]) + bn[0], (z[1] + v[1]) + bn[1], (z[2] + v[2]) + bn[2],
-                                 (z[3] + v[3]) + bn[3]};
-      } else if (mode == 2) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = pf_gelu(v[j] + bn[j]);
-        pf_frag_put4(F, MT, N / 32, m, n, v, bad);
-      } else {
-        const int D = N / 3, bi = m / P, pos = t0 + m % P;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] += bn[j];
-        if (n < D) {
-          *(vh_f32x4*)(out + (size_t)m * ldo + n) = vh_f32x4{v[0], v[1], v[2], v[3]};
-        } else if (pos >= 0 && pos < tmax) {
-          const size_t at = ((size_t)(bi * L + layer) * tmax + pos) * D + (n % D);
-          *(vh_u32x2*)((n < 2 * D ? kc : vc) + at) =
-              vh_u32x2{f2h(v[0]) | ((unsigned)f2h(v[1]) << 16), f2h(v[2]) | ((unsigned)f2h(v[3]) << 16)};
-        }
+      for (int j = 0; j < 4; ++j) v[j] += bn[b][j];
+      if (nt < D) {
+        *(vh_f32x4*)(out + (size_t)m * ldo + nt + 4 * q) = v;
+      } else if (cached) {
+        vh_half* c = (nt < 2 * D ? kc + (nt - D) : vc + (nt - 2 * D)) + row;
+        *(vh_u32x2*)c = vh_u32x2{f2h(v[0]) | ((unsigned)f2h(v[1]) << 16), f2h(v[2]) | ((unsigned)f2h(v[3]) << 16)};
       }
     }
   }
-  if (bad) stc_u(err, VH_ERR_RANGE);
 }
 
 // Ring: NR stages of S k-steps of 32 in flight in registers before they go to
@@ -314,6 +376,15 @@ __device__ __forceinline__ void pf_pgemm_ring(
 // fragments go from LDS into a second register set, the stage after that from
 // registers into LDS and the one after from the caches into registers, so no
 // wave waits for LDS between its products.
+// The block barrier of the loop is in builtins the compiler counts waits by: it
+// then knows that the fragments read before it have arrived, and does not
+// wait for the next ones at the first product that uses the former.
+__device__ __forceinline__ void pf_pipe_sync() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xc07f);          // lgkmcnt(0): this wave's LDS reads and writes are done
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 template <int TM, int TN, int WM, int WN>
 __device__ __forceinline__ void pf_pgemm_pipe(
     const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int MT, int KT, int NT, int ks,
@@ -378,11 +449,11 @@ __device__ __forceinline__ void pf_pgemm_pipe(
   gload(0);
   put(0);
   if (1 < ns) gload(1);
-  vh_lds_sync();
+  pf_pipe_sync();
   frags(w[0], x[0], 0);
   if (1 < ns) put(1);
   if (2 < ns) gload(2);
-  vh_lds_sync();
+  pf_pipe_sync();
   for (int cc = 0; cc < ns; cc += 2) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -399,7 +470,7 @@ __device__ __forceinline__ void pf_pgemm_pipe(
       __builtin_amdgcn_sched_barrier(0);
       mma(w[u], x[u], TM / 2, TM);
       __builtin_amdgcn_sched_barrier(0);
-      vh_lds_sync();
+      pf_pipe_sync();
     }
   }
   pf_pgemm_out<TM, TN>(ah, al, mt0 + wm * TM, nt0 + wn * TN, part, ks, MT, bias, M, N, mode, out, ldo, kc, vc, P, tp,

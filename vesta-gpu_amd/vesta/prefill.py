@@ -88,25 +88,29 @@ def _mtiles(rows: int) -> int:
 def pgemm_us(name, M, N, K, ks):
     """Estimated time of a product of more than FEW_ROWS rows, in us: a fixed
     part, and for each 32-deep k-step of a block a time by how many blocks a
-    CU gets (r). Fitted to measurements at the products of the three models
-    from 65 to 24576 rows, which it gives within about 15%; e.g. (measured,
-    us) qkv of GPT-2 small at 128 rows 6.9 / 12.4 / 27.8 in 32 x 64 / 64 x 128 /
-    128 x 256 tiles, at 1024 rows 18.4 / 18.6 / 28.3, at 24576 rows 284 / 216
-    (four waves: 189) / 192; narrowing of XL at 8192 rows 560 / 408 (384) / 336."""
+    CU gets (r). Fitted to the products of the three models at 65 to 24576
+    rows, timed alone and inside whole prefills (where weights and activations
+    come from farther away): the choice by it is within 2% of the fastest on
+    average, some 20-30% off at a few row counts (small at 1024 rows, the
+    out-projection: 9.2 against 7.5 us); e.g. (measured alone,
+    us) qkv of GPT-2 small at 128 rows 6.6 / 11.1 / 22.6 in 32 x 64 / 64 x 128 /
+    128 x 256 tiles, at 1024 rows 17.8 / 18.5 (four waves: 17.4) / 24.1, at
+    24576 rows 280 / 207 (177) / 174; narrowing of XL at 8192 rows 552 / 405
+    (373) / 332."""
     bm, bn, _ = PG_TILES[name]
     b = -(-M // (16 * bm)) * -(-N // (16 * bn)) * ks / 256
     k = K / 32 / ks
-    r = math.ceil(b) if b <= 4 else b
+    r = math.ceil(b) if b <= 6 else b
     if name == 'pf_pgemm128':                           # one block per CU at a time
-        us = math.ceil(b) * (11 + 0.76 * k)
+        us = math.ceil(b) * (8.61 + 0.719 * k)
     elif name == 'pf_pgemm64':
-        us = 3.5 + k * max(0.37, 0.31 * r)
-    elif name == 'pf_pgemm64w':
-        us = 3.5 + k * max(0.50, 0.15 + 0.30 * r)
+        us = 2.25 + k * max(0.448, 0.295 * r) + 1.14 * b
+    elif name == 'pf_pgemm64w':                         # (reads its weights through L2, dearer where they are deep)
+        us = 2.39 + k * max(0.662, 0.309 * r * (1 + 8.7e-6 * K) - 0.021)
     else:
-        us = 3 + k * max(0.165, 0.12 * r)
-    # the parts of a split fold are stored and read back
-    return us + (1 + ks * M * N * 8 / 5e6 if ks > 1 else 0)
+        us = 3.43 + k * max(0.162, 0.11 * r * (1 + 8.9e-6 * K))
+    # the parts of a split fold are stored and read back (by the launch that makes the LayerNorm either way)
+    return us + ((1.43 * ks - 0.665) * M * N * 1e-6 - 0.25 if ks > 1 else 0)
 
 
 def pgemm_plan(M, N, K, split):
