@@ -598,7 +598,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_embed_ln(const int* __restr
 // registers between the two.
 extern "C" __global__ __launch_bounds__(256) void pf_reduce_ln(
     const float* __restrict__ ws, int ksplit, const vh_half* __restrict__ bias, int M, int D,
-    float* __restrict__ Z, int ldz, const vh_half* __restrict__ w, const vh_half* __restrict__ b, vh_half* __restrict__ F,
+    float* __restrict__ Z, const vh_half* __restrict__ w, const vh_half* __restrict__ b, vh_half* __restrict__ F,
     int MT, unsigned* __restrict__ err) {
   __shared__ float red[VNWAVE];
   const int m = blockIdx.x, k8 = 8 * threadIdx.x;
@@ -606,7 +606,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_ln(
   float v[8] = {}, zr[8] = {}, bn[8] = {}, wv[8] = {}, bv[8] = {};
   if (in) {
     pf_ld8f(ws + (size_t)m * D + k8, v);
-    pf_ld8f(Z + (size_t)m * ldz + k8, zr);
+    pf_ld8f(Z + (size_t)m * D + k8, zr);
     if (bias) unpack8(ld16(bias + k8), bn);
     unpack8(ld16(w + k8), wv);
     unpack8(ld16(b + k8), bv);
@@ -623,7 +623,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_ln(
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (zr[j] + v[j]) + bn[j];
-    float* zp = Z + (size_t)m * ldz + k8;
+    float* zp = Z + (size_t)m * D + k8;
     *(vh_f32x4*)zp = vh_f32x4{v[0], v[1], v[2], v[3]};
     *(vh_f32x4*)(zp + 4) = vh_f32x4{v[4], v[5], v[6], v[7]};
   }
@@ -1405,9 +1405,8 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
 PF_ATTN(pf_attn, false)
 PF_ATTN(pf_attn16, true)
 
-// One query per row (a decode step, or the last of a row's P positions): one
-// block per (row m, head h; queries ldq apart), every thread of the block on
-// the positions 0 .. t0 + ahead, so that a step's cache rows
+// One position per row (a decode step): one block per (row m, head h), every
+// thread of the block on the positions 0 .. t0, so that a step's cache rows
 // are read with a block's worth of loads in flight instead of a wave's. Each
 // score is read by eight lanes, one 16-byte piece of the position's key row
 // each (so a wave's load covers eight whole rows), the eight partial dots
@@ -1422,7 +1421,7 @@ PF_ATTN(pf_attn16, true)
 // attention launch 19.3 -> 17.8 us; XL at 64 rows 3.023 -> 3.000).
 extern "C" __global__ __launch_bounds__(256) void pf_attn1(const float* __restrict__ Q, const vh_half* __restrict__ kc,
                                                             const vh_half* __restrict__ vc,
-                                                            int ldq, int ahead, const int* __restrict__ tp, int layer, int L, int tmax,
+                                                            const int* __restrict__ tp, int layer, int L, int tmax,
                                                             int H, vh_half* __restrict__ F, int MT,
                                                             unsigned* __restrict__ err) {
   __shared__ float qs[PF_E];
@@ -1442,7 +1441,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1(const float* __restri
   const int g = tid >> 3, b8 = tid & 7;
   float qv[8];
   {
-    const float* qp = Q + (size_t)m * ldq + h * PF_E + 8 * b8;
+    const float* qp = Q + (size_t)m * D + h * PF_E + 8 * b8;
     const vh_f32x4 q0 = *(const vh_f32x4*)qp, q1 = *(const vh_f32x4*)(qp + 4);
     qv[0] = q0[0]; qv[1] = q0[1]; qv[2] = q0[2]; qv[3] = q0[3];
     qv[4] = q1[0]; qv[5] = q1[1]; qv[6] = q1[2]; qv[7] = q1[3];
@@ -1454,7 +1453,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1(const float* __restri
     kr[u] = ld16_nt(kc + base + (size_t)s * D + 8 * b8);
   }
   __builtin_amdgcn_sched_barrier(0);    // the loads above issued before the position is waited for
-  const int at = *tp + ahead;
+  const int at = *tp;
   const int pos = at < tmax ? at : tmax - 1;
   float mx = -INFINITY;
   int s0 = g;
@@ -1568,7 +1567,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1(const float* __restri
 // loaded but not used.
 extern "C" __global__ __launch_bounds__(256) void pf_attn1s(const float* __restrict__ Q, const vh_half* __restrict__ kc,
                                                              const vh_half* __restrict__ vc,
-                                                             int ldq, int ahead, const int* __restrict__ tp, int layer, int L, int tmax,
+                                                             const int* __restrict__ tp, int layer, int L, int tmax,
                                                              int H, vh_half* __restrict__ F, int MT,
                                                              unsigned* __restrict__ err) {
   __shared__ float qs[PF_E];
@@ -1581,7 +1580,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1s(const float* __restr
   const int g = tid >> 3, b8 = tid & 7;
   float qv[8];
   {
-    const float* qp = Q + (size_t)m * ldq + h * PF_E + 8 * b8;
+    const float* qp = Q + (size_t)m * D + h * PF_E + 8 * b8;
     const vh_f32x4 q0 = *(const vh_f32x4*)qp, q1 = *(const vh_f32x4*)(qp + 4);
     qv[0] = q0[0]; qv[1] = q0[1]; qv[2] = q0[2]; qv[3] = q0[3];
     qv[4] = q1[0]; qv[5] = q1[1]; qv[6] = q1[2]; qv[7] = q1[3];
@@ -1595,7 +1594,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attn1s(const float* __restr
     vr[u] = ld16_nt(vc + at8);
   }
   __builtin_amdgcn_sched_barrier(0);    // the loads above issued before the position is waited for
-  const int at = *tp + ahead;
+  const int at = *tp;
   const int pos = at < tmax ? at : tmax - 1;
   float mx = -INFINITY, sm = 0.0f, o[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   int s0 = g;

@@ -26,7 +26,6 @@ from __future__ import annotations
 import ctypes
 import math
 from pathlib import Path
-from types import SimpleNamespace
 
 from .launch import compile_code, lib, ok, track, unload
 
@@ -251,9 +250,8 @@ class Prefill:
         """Activation buffers for M rows (one set per row count, kept): the
         residual Z, the queries Q, and the fragment-order activations AF of
         the products over d (LayerNorm and attention outputs) and GF of the
-        one over the feed-forward width (GELU outputs), and CF like AF for
-        each row's last position. These are zeroed once: rows past M are
-        never written (in GF, by the last layer's fewer rows, never read)."""
+        one over the feed-forward width (GELU outputs). These are zeroed
+        once: rows past M are never written."""
         import torch
         if M not in self._bufs:
             m = self.m
@@ -304,7 +302,7 @@ class Prefill:
             raise ValueError(f'decode product {wname}: operands smaller than {M}x{K} activations / {N}x{K} weights')
         if mode == MODE_GELU and (N % 32 or F is None or F.numel() < 2 * 16 * mt * N):
             raise ValueError(f'decode product {wname}: GELU output needs a fragment buffer of {M}x{N}, N % 32 == 0')
-        if mode in (MODE_PLAIN, MODE_RESID, MODE_QKV) and out.numel() < (M - 1) * ldo + (N // 3 if mode == MODE_QKV else N):
+        if mode in (MODE_PLAIN, MODE_RESID, MODE_QKV) and out.numel() < M * ldo:
             raise ValueError(f'decode product {wname}: output smaller than {M} rows of {ldo}')
         t_args = [_p(m.keys), _p(m.vals), _i(P), _p(m.t), _i(layer or 0), _i(m.L), _i(m.tmax)]
         self._launch(f'pf_mgemm{mt}' + ('n' if self._weights_nt() else ''), nb * ks,
@@ -319,7 +317,7 @@ class Prefill:
         m = self.m
         KT, NT, MT = K // 32, -(-N // 16), _mtiles(M)
         if ks is None:
-            name, ks = pgemm_plan(M, N, K, mode == MODE_RESID and ln is not None)
+            name, ks = pgemm_plan(M, N, K, mode == MODE_RESID and ln is not None and ldo == N)
         else:
             name = 'pf_pgemm32'
         ws = self._workspace(ks * M * N) if ks > 1 else None
@@ -352,8 +350,8 @@ class Prefill:
             return False
         if mode == MODE_RESID and ln is not None:
             w, b, Fo = ln
-            self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _i(ldo), _p(w),
-                                             _p(b), _p(Fo), _i(MT), _p(self.err)])
+            self._launch('pf_reduce_ln', M, [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(out), _p(w), _p(b), _p(Fo),
+                                             _i(MT), _p(self.err)])
             return True
         if mode == MODE_GELU:
             self._launch('pf_reduce_frag', -(-M * (N // 8) // BLOCK), [_p(ws), _i(ks), _p(bias), _i(M), _i(N), _p(F),
@@ -486,56 +484,48 @@ class Prefill:
         F = m.W['fcw'].shape[2]
         V = m.W['wte'].shape[0]
         W = m.W
-        Z, Q, err = buf['Z'], buf['Q'], self.err
+        Z, Q, AF, GF, err = buf['Z'], buf['Q'], buf['AF'], buf['GF'], self.err
+        mt = _mtiles(M)
         fixed = ordered(P, L)
-        # what the products of a layer work on: all M rows; in the last layer, once its cache rows are written, only
-        # each row's last position goes on (rows P - 1, 2 P - 1, .. of Z)
-        every = SimpleNamespace(M=M, P=P, A=buf['AF'], Z=Z, ldz=D, row0=0, stride=1)
-        tail = every if P == 1 or fixed else SimpleNamespace(M=B, P=P, A=buf['CF'], Z=Z.view(-1)[(P - 1) * D:],
-                                                             ldz=P * D, row0=P - 1, stride=P)
-        GF = buf['GF']
 
-        def norm(r, w, b, to=None):
-            to, mt = r.A if to is None else to, _mtiles(r.M)
-            if r.M >= LNM_ROWS and r.stride == 1:
-                self._launch('pf_lnm8' if D <= 1024 else 'pf_lnm16', -(-r.M // 16),
-                             [_p(Z), _i(r.M), _i(D), _p(w), _p(b), _p(to), _i(mt), _p(err)])
-            else:
-                self._launch('pf_ln', r.M, [_p(Z), _i(r.row0), _i(r.stride), _p(w), _p(b), _i(D), _p(to), _i(mt),
-                                            _p(err)])
+        def norm(w, b, to, rows, row0=0, stride=1):
+            if rows >= LNM_ROWS and stride == 1:
+                self._launch('pf_lnm8' if D <= 1024 else 'pf_lnm16', -(-rows // 16),
+                             [_p(Z), _i(rows), _i(D), _p(w), _p(b), _p(to), _i(_mtiles(rows)), _p(err)])
+                return
+            self._launch('pf_ln', rows, [_p(Z), _i(row0), _i(stride), _p(w), _p(b), _i(D), _p(to), _i(_mtiles(rows)),
+                                         _p(err)])
         self._launch('pf_embed_ln', M, [_p(tok), _i(P), _p(m.t), _p(W['wte']), _p(W['wpe']), _p(Z), _i(D), _i(V),
-                                        _i(W['wpe'].shape[0]), _p(W['ln1w'][0]), _p(W['ln1b'][0]), _p(every.A),
-                                        _i(_mtiles(M)), _p(err)])
+                                        _i(W['wpe'].shape[0]), _p(W['ln1w'][0]), _p(W['ln1b'][0]), _p(AF), _i(mt),
+                                        _p(err)])
         for layer in range(L):
             def lw(name, layer=layer):
                 return W[name][layer]
-            last = layer + 1 == L
-            self._product(every.A, D, 'qkvw', layer, 3 * D, MODE_QKV, bias=lw('qkvb'), out=Q, ldo=D, M=M, P=P,
+            self._product(AF, D, 'qkvw', layer, 3 * D, MODE_QKV, bias=lw('qkvb'), out=Q, ldo=D, M=M, P=P,
                           ordered=fixed)
-            r = tail if last else every
-            cache, at = [_p(m.keys), _p(m.vals)], [_p(m.t), _i(layer), _i(L), _i(m.tmax), _i(H), _p(r.A),
-                                                   _i(_mtiles(r.M)), _p(err)]
-            if r.M == B:        # one query per row: a block per (row, head) (GPT-2 small, 32 rows, 1024 positions:
+            cache = [_p(Q), _p(m.keys), _p(m.vals)]
+            if P == 1:          # a block per (row, head) (GPT-2 small, 32 rows, 1024 positions:
                                 # 1.32 -> 1.07 ms per step against a wave per (row, head))
-                self._launch(self._attn1(), B * H, [_p(Q.view(-1)[(P - 1) * D:])] + cache + [_i(P * D), _i(P - 1)] + at)
+                self._launch(self._attn1(), B * H, cache + [_p(m.t), _i(layer), _i(L), _i(m.tmax), _i(H), _p(AF),
+                                                            _i(mt), _p(err)])
             else:
                 name, blocks = prefill_attn(B, P, H, fixed)
-                self._launch(name, 8 * -(-blocks // 8), [_p(Q)] + cache + [_i(B), _i(P)] + at)
-            if not self._product(r.A, D, 'ow', layer, D, MODE_RESID, bias=lw('ob'), out=r.Z, ldo=r.ldz,
-                                 ln=(lw('ln2w'), lw('ln2b'), r.A), M=r.M, ordered=fixed):
-                norm(r, lw('ln2w'), lw('ln2b'))
-            self._product(r.A, D, 'fcw', layer, F, MODE_GELU, bias=lw('fcb'), F=GF, M=r.M, ordered=fixed)
-            # the next layer's first norm, or the final one: of each row's last position, into CF
-            w, b = (W['lnfw'], W['lnfb']) if last else (lw('ln1w', layer + 1), lw('ln1b', layer + 1))
-            whole = not last or r.M == B
-            if not self._product(GF, F, 'pw', layer, D, MODE_RESID, bias=lw('pb'), out=r.Z, ldo=r.ldz,
-                                 ln=(w, b, r.A) if whole else None, M=r.M, ordered=fixed):
-                if whole:
-                    norm(r, w, b)
-                else:
-                    norm(SimpleNamespace(M=B, row0=P - 1, stride=P), w, b, buf['CF'])
-        head = every.A if P == 1 else buf['CF']
+                self._launch(name, 8 * -(-blocks // 8), cache + [_i(B), _i(P), _p(m.t), _i(layer), _i(L), _i(m.tmax),
+                                                                 _i(H), _p(AF), _i(mt), _p(err)])
+            if not self._product(AF, D, 'ow', layer, D, MODE_RESID, bias=lw('ob'), out=Z, ldo=D,
+                                 ln=(lw('ln2w'), lw('ln2b'), AF), M=M, ordered=fixed):
+                norm(lw('ln2w'), lw('ln2b'), AF, M)
+            self._product(AF, D, 'fcw', layer, F, MODE_GELU, bias=lw('fcb'), F=GF, M=M, ordered=fixed)
+            last = layer + 1 == L
+            nxt = (W['lnfw'], W['lnfb'], AF) if last else (lw('ln1w', layer + 1), lw('ln1b', layer + 1), AF)
+            normed = self._product(GF, F, 'pw', layer, D, MODE_RESID, bias=lw('pb'), out=Z, ldo=D,
+                                   ln=nxt if P == 1 or not last else None, M=M, ordered=fixed)
+            if not normed and not (last and P > 1):
+                norm(*nxt, M)
+        if P > 1:               # the final norm: each row's last position
+            norm(W['lnfw'], W['lnfb'], buf['CF'], B, P - 1, P)
         logit, nxt = m.logits(), m.next()
+        head = buf['CF'] if P > 1 else AF
         if B <= FEW_ROWS:
             self._mhead(head, D, V, logit, B)
         else:
