@@ -17,7 +17,9 @@
 // cache rounded to fp16 before attention reads it); products run on
 // v_mfma_f32_16x16x32_f16 with every activation split into two fp16 halves
 // (hi + lo / 2048: 22 significant bits at any magnitude), each half's products
-// accumulated in fp32 on its own and combined at the end.
+// accumulated in fp32 on its own and combined at the end. The attention's
+// contractions run there too, its queries and softmax weights in three planes
+// (pf_split24), so that they keep fp32's 24 bits.
 
 #define PF_E 64                 // head width
 
@@ -60,6 +62,25 @@ __device__ __forceinline__ void pf_frag_put4(vh_half* __restrict__ F, int MT, in
   const size_t at = (((size_t)(m >> 4) * KT + (k4 >> 5)) * 64 + ((k4 >> 3) & 3) * 16 + (m & 15)) * 8 + (k4 & 7);
   *(vh_u32x2*)(F + at) = __builtin_bit_cast(vh_u32x2, hi);
   *(vh_u32x2*)(F + (size_t)MT * KT * 512 + at) = __builtin_bit_cast(vh_u32x2, lo);
+}
+
+// Eight floats of at most 1 in magnitude as three fp16 planes v = hi + (lo +
+// tail) / 2^11, each plane what is left, cut off (not rounded) after 11 bits:
+// all 24 bits of a value down to 2^-12, smaller ones to 2^-35. The conversions
+// take two values an instruction.
+__device__ __forceinline__ void pf_split24(const float* v, vh_u32x4& hi, vh_u32x4& lo, vh_u32x4& tail) {
+  typedef __fp16 h2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const h2 h = __builtin_amdgcn_cvt_pkrtz(v[2 * j], v[2 * j + 1]);
+    const float r0 = fmaf((float)h[0], -VH_LO_SCALE, v[2 * j] * VH_LO_SCALE);
+    const float r1 = fmaf((float)h[1], -VH_LO_SCALE, v[2 * j + 1] * VH_LO_SCALE);
+    const h2 l = __builtin_amdgcn_cvt_pkrtz(r0, r1);
+    const h2 t = __builtin_amdgcn_cvt_pkrtz(r0 - (float)l[0], r1 - (float)l[1]);
+    hi[j] = __builtin_bit_cast(unsigned, h);
+    lo[j] = __builtin_bit_cast(unsigned, l);
+    tail[j] = __builtin_bit_cast(unsigned, t);
+  }
 }
 
 // ---------------------------------------------------------------- products
@@ -1082,15 +1103,23 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_frag(const float* __
 // first left them in: the instruction's fold position 8q + e of lane group q
 // stands for cache position 4q + e (e < 4) and 16 + 4q + e - 4 of a tile's 32,
 // and V is staged in that order. Queries (scaled by a power of two per query,
-// so that any fp32 magnitude splits) and softmax weights are split into fp16
-// halves like a product's activations (22 bits), each half in its own
-// accumulator. A score whose hi part is infinite is that infinity (the cache
-// may hold one, and 0 * inf of the lo part would make it a NaN).
+// so that any fp32 magnitude splits) and softmax weights go in as three fp16
+// planes (pf_split24: 24 bits), the two lower ones in one accumulator. The two
+// halves of a score's dims, and each tile's weighted values and weights, are
+// summed on their own and added in fp32 after, so that no sum is a chain over
+// all positions. Errors against 64 bits, relative (2-norm), fp32 throughout with
+// a wave per (query row, head) / halves of 22 bits in running accumulators / this:
+// GPT-2 small 1 x 37 7.5e-8 / 7.8e-8 / 7.3e-8, 2 x 768 1.03e-7 / 1.15e-7 / 8.7e-8,
+// 1 x 200 after 700 positions 1.93e-7 / 2.26e-7 / 1.2e-7, medium 3 x 333 after 100
+// 1.33e-7 / 1.50e-7 / 1.08e-7.
+// A score whose hi part is infinite is that infinity (the cache may hold one,
+// and 0 * inf of the lower parts would make it a NaN).
 // What bounds it: vector work on the scores (exponentials, maxima, splits;
-// about 3 x the matrix-core time); few queries: the chain of tiles, 1.3 us
-// each. GPT-2 small, 32 x 768: 134 us a layer against 1198 with a wave per
-// (query row, head), which read every cache row once per query; 8 x 128 6.9
-// against 19.7; medium 3 x 333 after 100 positions 59 -> 22.
+// about twice the matrix-core time); few queries: the chain of tiles, 1.6 us
+// each. GPT-2 small, 32 x 768: 161 us a layer (22-bit halves 140) against 1170
+// with a wave per (query row, head), which read every cache row once per query;
+// 8 x 128 7.5 (7.1) against 20.0; medium 3 x 333 after 100 positions 16.9 (15.0)
+// against 56.
 // F receives the head's output, row m, in fragment order.
 // One query over at most 64 positions by one wave, in fp32 throughout: eight
 // lanes per position for the dots (the partial dots added across them), a
@@ -1139,7 +1168,7 @@ __device__ __forceinline__ void pf_attn_short(const float* __restrict__ qp, cons
 // With SPLIT a block makes 16 queries: its waves take every fourth tile of
 // positions each, staged for themselves, and combine at the end: where few
 // queries would leave waves or most of the chip idle over a long cache
-// (GPT-2 small, 3 tokens after 900 positions: 21.6 -> 10.8 us a launch). A
+// (GPT-2 small, 3 tokens after 900 positions: 25.1 -> 11.1 us a launch). A
 // prompt of at most PF_SHORT tokens that sees at most 64 positions goes a
 // query at a time instead (pf_attn_short; no slower: one tile has no parts to
 // split).
@@ -1183,8 +1212,8 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
     if (bad) stc_u(err, VH_ERR_RANGE);
     return;
   }
-  // the query, scaled to below 1 by 2^-e, in halves: dims 32 s + 8 q .. + 7
-  vh_u32x4 qh[2], ql[2];
+  // the query, scaled to below 1 by 2^-e, in its three planes: dims 32 s + 8 q .. + 7
+  vh_u32x4 qh[2], ql[2], qt[2];
   float k2;                                                        // 2^e / 8 log2(e): scores in powers of 2
   {
     const float* qp = Q + ((size_t)b * P + min(pq, P - 1)) * D + h * PF_E + 8 * q;
@@ -1209,7 +1238,7 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[s][j] = __builtin_ldexpf(v[s][j], -e);
-      vh_split8s(v[s], qh[s], ql[s]);
+      pf_split24(v[s], qh[s], ql[s], qt[s]);
     }
     k2 = __builtin_ldexpf(0.125f * 1.44269504088896341f, e);
   }
@@ -1252,9 +1281,7 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
       }
     }
   };
-  vh_f32x4 oh[4], ol[4];
-#pragma unroll
-  for (int d = 0; d < 4; ++d) oh[d] = ol[d] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float o[4][4] = {};                    // weighted values: dim tile, dim of it
   float m2 = -INFINITY, sum = 0.0f;      // largest score in powers of 2; the sum of this lane's positions
   if constexpr (SPLIT) {
     if (wave < nt) gload(wave);
@@ -1281,14 +1308,15 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
     vh_f32x4 sh[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      vh_f32x4 sl = {0.0f, 0.0f, 0.0f, 0.0f};
-      sh[i] = sl;
+      vh_f32x4 h[2] = {}, sl = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const vh_u32x4 kf = K[(2 * i + k) * 64 + lane];
-        sh[i] = vh_mfma(kf, qh[k], sh[i]);
+        h[k] = vh_mfma(kf, qh[k], h[k]);
         sl = vh_mfma(kf, ql[k], sl);
+        sl = vh_mfma(kf, qt[k], sl);
       }
+      sh[i] = vh_f32x4{h[0][0] + h[1][0], h[0][1] + h[1][1], h[0][2] + h[1][2], h[0][3] + h[1][3]};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         s[i][j] = vh_hilo(sh[i][j], sl[j]);
@@ -1314,48 +1342,35 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
     bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
     const float n2 = fmaxf(m2, bm * k2);
     const float ref = n2 == -INFINITY ? 0.0f : n2;                 // no score above -inf yet: all weights 0
-    if (__any(n2 != m2)) {
-      const float c = __builtin_amdgcn_exp2f(m2 - ref);            // 0 while m2 is -inf
-      sum *= c;
-#pragma unroll
-      for (int d = 0; d < 4; ++d)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          oh[d][j] *= c;
-          ol[d][j] *= c;
-        }
-      m2 = n2;
-    }
-    vh_u32x4 ph[2], pl[2];
+    const float c = __builtin_amdgcn_exp2f(m2 - ref);              // 0 while m2 is -inf
+    m2 = n2;
+    vh_u32x4 ph[2], pl[2], pt[2];
+    float ts[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      vh_h8 hi, lo;
+      float w[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float w = __builtin_amdgcn_exp2f(fmaf(s[2 * k + (j >> 2)][j & 3], k2, -ref));
-        sum += w;
-        hi[j] = (_Float16)w;
-        lo[j] = (_Float16)fmaf((float)hi[j], -VH_LO_SCALE, w * VH_LO_SCALE);     // (w - hi) 2^11, exact
-      }
-      ph[k] = __builtin_bit_cast(vh_u32x4, hi);
-      pl[k] = __builtin_bit_cast(vh_u32x4, lo);
+      for (int j = 0; j < 8; ++j) w[j] = __builtin_amdgcn_exp2f(fmaf(s[2 * k + (j >> 2)][j & 3], k2, -ref));
+      ts[k] = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+      pf_split24(w, ph[k], pl[k], pt[k]);
     }
+    sum = fmaf(sum, c, ts[0] + ts[1]);
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
+    for (int d = 0; d < 4; ++d) {
+      vh_f32x4 th = {0.0f, 0.0f, 0.0f, 0.0f}, tl = th;
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const vh_u32x4 vf = V[(2 * d + k) * 64 + lane];
-        oh[d] = vh_mfma(vf, ph[k], oh[d]);
-        ol[d] = vh_mfma(vf, pl[k], ol[d]);
+        th = vh_mfma(vf, ph[k], th);
+        tl = vh_mfma(vf, pl[k], tl);
+        tl = vh_mfma(vf, pt[k], tl);
       }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[d][j] = fmaf(o[d][j], c, vh_hilo(th[j], tl[j]));
+    }
   }
   sum += __shfl_xor(sum, 16, 64);
   sum += __shfl_xor(sum, 32, 64);
-  float o[4][4];
-#pragma unroll
-  for (int d = 0; d < 4; ++d)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[d][j] = vh_hilo(oh[d][j], ol[d][j]);
   if constexpr (SPLIT) {
     // each wave's maximum, sum and output rescaled to the common maximum and
     // added in wave order; wave w then writes dim tile w

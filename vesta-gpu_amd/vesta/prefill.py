@@ -62,8 +62,8 @@ LNM_ROWS = 1536               # LayerNorms of at least this many rows take a blo
 ORDERED_TOKENS, ORDERED_LAYERS = 8, 24      # see ordered()
 ATTN_SPLIT_BLOCKS = 512       # prefill attention with at most this many blocks of 16 queries (two per CU, all
                               # resident) splits each one's positions over its waves (pf_attn16). us a launch, pf_attn
-                              # / pf_attn16, GPT-2 small: 1 x 200 after 700 positions (156 such blocks) 22.0 / 10.6,
-                              # 20 x 32 after 365 (480) 13.3 / 11.7, 60 x 3 (720) 6.3 / 8.2, 8 x 128 (768) 6.9 / 10.3
+                              # / pf_attn16, GPT-2 small: 1 x 200 after 700 positions (156 such blocks) 25.3 / 10.9,
+                              # 20 x 32 after 365 (480) 14.6 / 11.9, 60 x 3 (720) 6.6 / 6.8, 8 x 128 (768) 7.5 / 10.9
 ATTN_ONE_PASS_BLOCKS = 1024   # decode passes with at most this many (row, head) blocks read each cache row in
                               # one pass (pf_attn1s), more in two (pf_attn1: keys, then values; fewer
                               # registers, more blocks resident). Same box, two -> one pass: small 16 / 24 rows
