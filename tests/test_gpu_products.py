@@ -191,3 +191,56 @@ def test_up_to_eight_rows_compute_what_more_rows_compute(shape):
     for rows, g in zip((8, 3, 1), got[1:]):
         for a, b in zip(g, got[0]):
             assert torch.equal(a, b[:rows])
+
+
+def _lnm_and_ln(e, X, w, b):
+    """The LayerNorm of X's rows by a block per 16 rows and by a block per row, as fp32 pairs of planes."""
+    import torch
+    from vesta import prefill as pf
+    M, D = X.shape
+    p, i, MT = pf._p, pf._i, pf._mtiles(M)
+    out = []
+    for name in ('pf_lnm8' if D <= 1024 else 'pf_lnm16', 'pf_ln'):
+        F = torch.zeros(2 * 16 * MT * D, dtype=torch.float16, device='cuda')
+        e._plan = []
+        if name == 'pf_ln':
+            e._launch(name, M, [p(X), i(0), i(1), p(w), p(b), i(D), p(F), i(MT), p(e.err)])
+        else:
+            e._launch(name, -(-M // 16), [p(X), i(M), i(D), p(w), p(b), p(F), i(MT), p(e.err)])
+        plan, e._plan = e._plan, []
+        e._replay(plan)
+        out.append(_unfrag(F, M, D))
+    return out
+
+
+@pytest.mark.parametrize('D', [768, 1024, 1600, 2048])
+@pytest.mark.parametrize('mean', [0.0, 30.0])
+def test_layer_norm_of_many_rows_is_as_exact_as_of_few(engine, D, mean):
+    """Both kernels' distances from 64 bits (2-norm) over 999 rows. Distances are over 999 * D values, but the error of a
+    row's mean is common to its D values: 999 samples of each, 2.2% of a root mean square, 3.2% of the quotient of two,
+    10% three times that."""
+    import torch
+    gen = torch.Generator(device='cuda').manual_seed(D)
+    X, w, b = (torch.randn(*s, generator=gen, device='cuda') for s in ((999, D), (D,), (D,)))
+    X, w, b = X + mean, (1 + 0.1 * w).half(), (0.02 * b).half()
+    c = X.double() - X.double().mean(-1, keepdim=True)
+    want = c / torch.sqrt((c * c).mean(-1, keepdim=True) + 1e-5) * w.double() + b.double()
+    many, few = ((y - want).norm().item() for y in _lnm_and_ln(engine._pf, X, w, b))
+    print(f'{D} wide, mean {mean}: {many / want.norm().item():.3e}, a block per row {few / want.norm().item():.3e}')
+    assert many <= 1.1 * few
+    engine.check()
+
+
+@pytest.mark.parametrize('D', [768, 1600, 2048])
+@pytest.mark.parametrize('size', [1e15, 1e18, 4e18, 1e20, 1e30])
+def test_layer_norm_of_many_rows_takes_what_of_few_takes(engine, D, size):
+    """Rows whose squares reach, and pass, the end of fp32's range: what a block per row accepts (its biases, where the
+    variance is infinite) a block per 16 rows accepts, with the same result to their sums' rounding."""
+    import torch
+    gen = torch.Generator(device='cuda').manual_seed(D)
+    X, w, b = (torch.randn(*s, generator=gen, device='cuda') for s in ((33, D), (D,), (D,)))
+    X[::2] = X[::2] * size                                       # large rows beside small ones
+    X[6, 1:] = 0                                                 # one value alone
+    many, few = _lnm_and_ln(engine._pf, X, w.half(), b.half())
+    engine.check()
+    _close(many, few, (2.0 ** -20 + D ** 0.5 * 2.0 ** -23) * (many.abs() + few.abs() + 1))

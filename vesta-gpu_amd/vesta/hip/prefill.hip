@@ -655,10 +655,20 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_ln(
 // wave w holding row r's values 8 (16 i + 4 w + q) .. + 7, i < NP (D <= 128 NP),
 // so that a wave stores a whole fragment, one contiguous kilobyte, where a
 // block per row stores 16 bytes of each 256 and eight XCDs write each line.
-// Sums per lane, over the lanes of a row, then over the waves. Bound by the
-// bytes where there are blocks enough: 24576 rows of 768 66.2 -> 25.7 us (5.9
-// TB/s), 8192 of 1600 46.7 -> 21.1; 2048 of 768 8.9 -> 7.5; at 999 rows 6.4
-// against 7.0 and below, the block per row is faster.
+// Sums pairwise over a lane's eight values (pf_sum8), then over its pieces;
+// divided by D there, where a rounding is a sixteenth of one of the whole mean;
+// then over the lanes of a row and pairwise over the waves: 0.77-1.01 times
+// pf_ln's distance from 64 bits at a mean of 30 deviations (one running sum
+// divided at the end 1.5), 0.99-1.01 at none. pf_sum8 scales its terms by 2^-11
+// (D <= 2048), where pf_ln divides each by D: exact, and a row overflows here if
+// it does there (a variance beyond fp32 leaves the biases in both).
+// Bound by the bytes where there are blocks enough: 24576 rows of 768 65.8 ->
+// 25.6 us (5.9 TB/s), 8192 of 1600 46.6 -> 20.8; 2048 of 768 8.7 -> 7.7; at 999
+// rows 6.3 against 7.3 and below, the block per row is faster.
+__device__ __forceinline__ float pf_sum8(const float* v) {         // their sum, times 2^-11
+  constexpr float c = 1.0f / 2048.0f;
+  return (fmaf(v[0], c, v[1] * c) + fmaf(v[2], c, v[3] * c)) + (fmaf(v[4], c, v[5] * c) + fmaf(v[6], c, v[7] * c));
+}
 template <int NP>
 __device__ __forceinline__ void pf_lnm_body(const float* __restrict__ X, int M, int D, const vh_half* __restrict__ w,
                                             const vh_half* __restrict__ b, vh_half* __restrict__ F, int MT,
@@ -675,32 +685,30 @@ __device__ __forceinline__ void pf_lnm_body(const float* __restrict__ X, int M, 
   float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < NP; ++i)
-    if (pc0 + 16 * i < np)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) s += v[i][j];
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
-  if (lane < 16) red[0][wave][r] = s;
-  vh_lds_sync();
-  s = 0.0f;
-#pragma unroll
-  for (int k = 0; k < VNWAVE; ++k) s += red[0][k][r];
-  const float mean = s / (float)D;
+    if (pc0 + 16 * i < np) s += pf_sum8(v[i]);
+  const float d2 = (float)D / 2048.0f;
+  auto row_sum = [&](float p, float (*part)[16]) {                 // the lanes' sums p over the row, / D
+    p /= d2;
+    p += __shfl_xor(p, 16, 64);
+    p += __shfl_xor(p, 32, 64);
+    if (lane < 16) part[wave][r] = p;
+    vh_lds_sync();
+    static_assert(VNWAVE == 4, "pairwise over the waves");
+    return (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
+  };
+  const float mean = row_sum(s, red[0]);
   s = 0.0f;
 #pragma unroll
   for (int i = 0; i < NP; ++i)
-    if (pc0 + 16 * i < np)
+    if (pc0 + 16 * i < np) {
+      float u[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s = fmaf(v[i][j] - mean, v[i][j] - mean, s);
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
-  if (lane < 16) red[1][wave][r] = s;
-  vh_lds_sync();
-  s = 0.0f;
-#pragma unroll
-  for (int k = 0; k < VNWAVE; ++k) s += red[1][k][r];
+      for (int j = 0; j < 8; ++j) u[j] = (v[i][j] - mean) * (v[i][j] - mean);
+      s += pf_sum8(u);
+    }
+  float sd = sqrtf(row_sum(s, red[1]) + 0.00001f), rs = 1.0f / sd;
   if (!live) return;
-  const float sd = sqrtf(s / (float)D + 0.00001f), rs = 1.0f / sd;
+  if (sd == INFINITY) sd = 1.0f, rs = 0.0f;                        // x / inf by vh_divr's two products
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < NP; ++i) {

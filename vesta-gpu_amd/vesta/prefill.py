@@ -57,8 +57,8 @@ MEM_CACHE_BYTES = 256 << 20   # the device's memory-side cache: decode products 
                               # steps, nontemporal there: 32 rows 0.548 -> 0.553)
 WORKSPACE_MIN = 8 << 20        # floats; a plan whose build outgrows the workspace is built twice (some ms of host time)
 LNM_ROWS = 1536               # LayerNorms of at least this many rows take a block per 16 rows (pf_lnm*; us a
-                              # launch, block per row / per 16 rows: 999 x 768 6.4 / 7.0, 2048 x 768 8.9 / 7.5, 999 x
-                              # 1600 8.7 / 12.1, 2048 x 1600 13.5 / 13.9, 4096 x 1600 24.6 / 16.0)
+                              # launch, block per row / per 16 rows: 999 x 768 6.3 / 7.3, 2048 x 768 8.7 / 7.7, 999 x
+                              # 1600 8.3 / 12.7, 2048 x 1600 13.0 / 13.7, 4096 x 1600 24.0 / 15.9)
 ORDERED_TOKENS, ORDERED_LAYERS = 8, 24      # see ordered()
 ATTN_SPLIT_BLOCKS = 512       # prefill attention with at most this many blocks of 16 queries (two per CU, all
                               # resident) splits each one's positions over its waves (pf_attn16). us a launch, pf_attn
