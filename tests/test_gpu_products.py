@@ -121,6 +121,36 @@ def test_products_match_64_bits(engine, monkeypatch, kernel, M):
     _close(out, A.double() @ w.t(), (A.double().abs() @ w.abs().t()) * (2.0 ** -22 + D * 2.0 ** -24))
 
 
+@pytest.mark.parametrize('K,apart', [(1024, 1.57), (3072, 2.34)])
+def test_a_long_fold_is_nearly_as_exact_as_a_short_one(engine, monkeypatch, K, apart):
+    """pf_pgemm32, which takes long folds whole at some hundred rows, sums 128 of them at a time. In rounding units, with
+    partial sums that grow as the square root of their length, c sums of s k-steps added in order are
+    (s + 1) / 2 - 1 / s + (c + 1) / 2 - 1 / c squared from 64 bits, relative to the result, plus what a k-step's own sums
+    leave; so with s = 4 a fold of 1024 is at most sqrt(6.6 / 3.25) = 1.43 times as far as one of 256, one of 3072 2.13
+    times (one running sum: measured 1.73 and 2.9). 10% for the samples and the model."""
+    import torch
+    from vesta import prefill as pf
+    m, e, M, N = engine, engine._pf, 129, 768
+    monkeypatch.setattr(pf, 'pgemm_plan', lambda *a: ('pf_pgemm32', 1))
+    off = []
+    for k in (256, K):
+        gen = torch.Generator(device='cuda').manual_seed(k)
+        A, w = (torch.randn(*s, generator=gen, device='cuda') for s in ((M, k), (N, k)))
+        w = (0.02 * w).half()
+        Wf = pf.frag_weights(w).contiguous()
+        monkeypatch.setattr(e, '_frag', lambda name: Wf)
+        out, F = torch.zeros(M, N, device='cuda'), _frag(A)
+        e._plan = []
+        e._pgemm(F, k, 'w', None, N, pf.MODE_PLAIN, out=out, ldo=N, M=M)
+        plan, e._plan = e._plan, []
+        e._replay(plan)
+        want = _unfrag(F, M, k) @ w.double().t()
+        off.append(((out.double() - want).norm() / want.norm()).item())
+    print(f'{K}: {off[1]:.3e}, 256: {off[0]:.3e}')
+    assert off[1] <= apart * off[0]
+    e.check()
+
+
 def test_more_than_64_rows_decode_and_prefill_like_fewer():
     """70 rows (products in output tiles, the output head too) against the same rows in a batch of 8:
     the same tokens where the margin is clear, logits within the engines' tolerance."""

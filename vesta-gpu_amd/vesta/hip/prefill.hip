@@ -288,8 +288,14 @@ __device__ __forceinline__ void pf_pgemm_out(
 // Ring: NR stages of S k-steps of 32 in flight in registers before they go to
 // LDS; with WDIR the weight fragments skip LDS and go from the caches straight
 // into each wave's registers one stage ahead (the WM waves that share them
-// meet in the CU's L1).
-template <int TM, int TN, int WM, int WN, int S, bool WDIR, int NR>
+// meet in the CU's L1). With ANEW the hi halves' sums start anew with each turn
+// of the loop (NR stages) and are added in fp32: a fold in one running sum is up
+// to 1.7 times further from 64 bits than in parts of 256, which is what few rows
+// get from the waves and the blocks that split their folds (pf_pgemm32, 128
+// rows, in one sum / anew every 128: 1024 deep 2.10e-7 / 1.08e-7). It costs 0-1%
+// (1024 x 2304 x 768 17.9 -> 18.0 us); sums twice as long, behind a condition,
+// 2%.
+template <int TM, int TN, int WM, int WN, int S, bool WDIR, int NR, bool ANEW>
 __device__ __forceinline__ void pf_pgemm_ring(
     const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int MT, int KT, int NT, int ks,
     const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,
@@ -319,11 +325,11 @@ __device__ __forceinline__ void pf_pgemm_ring(
       src[i] = Wf + ((size_t)min(nt0 + t, NT - 1) * KT + c0 * S + s) * 64 + lane;
     }
   }
-  vh_f32x4 ah[TM][TN], al[TM][TN];
+  vh_f32x4 ah[TM][TN], al[TM][TN], sum[TM][TN];
 #pragma unroll
   for (int a = 0; a < TM; ++a)
 #pragma unroll
-    for (int b = 0; b < TN; ++b) ah[a][b] = al[a][b] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int b = 0; b < TN; ++b) ah[a][b] = al[a][b] = sum[a][b] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   vh_u32x4 st[NR][PER];
   auto gload = [&](vh_u32x4 (&d)[PER], int c) {
 #pragma unroll
@@ -351,6 +357,11 @@ __device__ __forceinline__ void pf_pgemm_ring(
   vh_lds_sync();
   constexpr int U = NR == 1 ? 2 : NR;
   for (int cc = 0; cc < ns; cc += U) {
+    if constexpr (ANEW)
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) ah[a][b] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = cc + u;
@@ -388,9 +399,16 @@ __device__ __forceinline__ void pf_pgemm_ring(
       }
       vh_lds_sync();
     }
+    if constexpr (ANEW)
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+          sum[a][b] = vh_f32x4{sum[a][b][0] + ah[a][b][0], sum[a][b][1] + ah[a][b][1], sum[a][b][2] + ah[a][b][2],
+                               sum[a][b][3] + ah[a][b][3]};
   }
-  pf_pgemm_out<TM, TN>(ah, al, mt0 + wm * TM, nt0 + wn * TN, part, ks, MT, bias, M, N, mode, out, ldo, kc, vc, P, tp,
-                       layer, L, tmax, ws, F, err);
+  pf_pgemm_out<TM, TN>(ANEW ? sum : ah, al, mt0 + wm * TM, nt0 + wn * TN, part, ks, MT, bias, M, N, mode, out, ldo, kc,
+                       vc, P, tp, layer, L, tmax, ws, F, err);
 }
 
 // Pipe: one k-step a stage; while a stage's products run, the next stage's
@@ -508,8 +526,9 @@ __device__ __forceinline__ void pf_pgemm_pipe(
   }
 PF_PGEMM(pf_pgemm128, 512, 2, pf_pgemm_pipe<4, 4, 2, 4>)              // 128 x 256
 PF_PGEMM(pf_pgemm64, 512, 4, pf_pgemm_pipe<2, 2, 2, 4>)               // 64 x 128, eight waves
-PF_PGEMM(pf_pgemm64w, 256, 2, pf_pgemm_ring<2, 4, 2, 2, 1, true, 2>)  // 64 x 128, four waves
-PF_PGEMM(pf_pgemm32, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, 2>)  // 32 x 64
+PF_PGEMM(pf_pgemm64w, 256, 2, pf_pgemm_ring<2, 4, 2, 2, 1, true, 2, false>)  // 64 x 128, four waves
+PF_PGEMM(pf_pgemm32, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, 2, true>)   // 32 x 64
+PF_PGEMM(pf_pgemm32o, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, 2, false>) // 32 x 64, one sum a part
 
 // The parts of a split product added in part order, then the epilogue. One
 // thread per output value.

@@ -37,7 +37,7 @@ HEAD = 64
 KERNELS = ('pf_ln', 'pf_lnm8', 'pf_lnm16', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn16', 'pf_attn1', 'pf_argmax_part', 'pf_argmax',
            'pf_mgemm1', 'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n', 'pf_mgemm2n', 'pf_mgemm4n', 'pf_reduce_frag', 'pf_attn1s',
            'pf_mhead1', 'pf_mhead2', 'pf_mhead4', 'pf_embed_ln', 'pf_pgemm128', 'pf_pgemm64',
-           'pf_pgemm64w', 'pf_pgemm32')
+           'pf_pgemm64w', 'pf_pgemm32', 'pf_pgemm32o')
 ARGMAX_SPLIT = 32             # blocks per row of the output-head argmax (same box, 16 -> 32: GPT-2 small 32 rows
                               # 547.6 -> 545.8 us per step, 8 rows 396.3 -> 395.5, XL 64 rows even)
 # output tiles of the products beyond FEW_ROWS rows: 16-row tiles, 16-column tiles and waves of a block
@@ -313,13 +313,15 @@ class Prefill:
     def _pgemm(self, Af, K, wname, layer, N, mode, bias=None, out=None, ldo=0, F=None, ln=None, M=1, P=1, ks=None):
         """One product of any number of rows (``pf_pgemm*``), as ``_mgemm``.
         With ``ks`` None only a residual product with a LayerNorm after it
-        splits its fold (its reduction adds no launch); else in ``ks`` parts."""
+        splits its fold (its reduction adds no launch); else it is made in
+        ``ks`` parts, each part's sum whole (``pf_pgemm32o``)."""
         m = self.m
         KT, NT, MT = K // 32, -(-N // 16), _mtiles(M)
         if ks is None:
             name, ks = pgemm_plan(M, N, K, mode == MODE_RESID and ln is not None and ldo == N)
+            bm, bn, waves = PG_TILES[name]
         else:
-            name = 'pf_pgemm32'
+            name, (bm, bn, waves) = 'pf_pgemm32o', PG_TILES['pf_pgemm32']
         ws = self._workspace(ks * M * N) if ks > 1 else None
         Wf = self._frag(wname)
         Wf = Wf[layer] if layer is not None else Wf
@@ -334,7 +336,6 @@ class Prefill:
             raise ValueError(f'product {wname}: output smaller than {M} rows of {ldo}')
         if mode != MODE_PLAIN and (N % 64 or ldo % 4 or bias is None):
             raise ValueError(f'product {wname}: N={N} must be a multiple of 64, the output pitch of 4, with a bias')
-        bm, bn, waves = PG_TILES[name]
         tiles = -(-MT // bm) * -(-NT // bn) * ks
         self._launch(name, 8 * -(-tiles // 8),
                      [_p(Af), _p(Wf), _i(MT), _i(KT), _i(NT), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out),
