@@ -93,14 +93,29 @@ def test_prefill_attention_takes_any_query_magnitude(engine, kernel):
 
 
 @pytest.mark.parametrize('kernel', ['pf_attn', 'pf_attn16'])
-def test_a_key_of_minus_infinite_score_has_no_weight(engine, kernel):
-    """A cache row that overflowed fp16 in one key component: queries whose score there is -inf ignore it."""
+@pytest.mark.parametrize('q7', [-0.5, -0.3, -1e-9, -1e-30])
+def test_a_key_of_minus_infinite_score_has_no_weight(engine, kernel, q7):
+    """A cache row that overflowed fp16 in one key component: queries whose score there is -inf ignore it, whichever of
+    their component's planes are 0 (-0.5: all but the first; below 2^-25 of the largest: the first)."""
     P, t0 = 5, 90
     Q, k, v = _inputs(P, t0)
-    Q.view(B, P, H, 64)[..., 7] = -0.5                    # exact in fp16: its lo half is 0
+    Q.view(B, P, H, 64)[..., 7] = q7
     k[:, 1, 40, :, 7] = float('inf')
     _check(_run(engine, kernel, Q, k, v, t0, P), Q, k, v, t0, P)
     engine.check()
+
+
+@pytest.mark.parametrize('kernel', ['pf_attn', 'pf_attn16'])
+@pytest.mark.parametrize('q7', [0.5, 1e-9, 0.0])
+def test_an_infinite_or_undefined_score_is_refused(engine, kernel, q7):
+    """+inf (its weight is inf - inf) and 0 * inf: the outputs are no numbers, and the range word says so."""
+    P, t0 = 5, 90
+    Q, k, v = _inputs(P, t0)
+    Q.view(B, P, H, 64)[..., 7] = q7
+    k[:, 1, 40, :, 7] = float('inf')
+    assert _run(engine, kernel, Q, k, v, t0, P).isnan().all()
+    with pytest.raises(RuntimeError, match='fp16 range'):
+        engine.check()
 
 
 def _in_fp32(Q, k, v, t0, P):

@@ -1139,8 +1139,10 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_frag(const float* __
 // GPT-2 small 1 x 37 7.5e-8 / 7.8e-8 / 7.3e-8, 2 x 768 1.03e-7 / 1.15e-7 / 8.7e-8,
 // 1 x 200 after 700 positions 1.93e-7 / 2.26e-7 / 1.2e-7, medium 3 x 333 after 100
 // 1.33e-7 / 1.50e-7 / 1.08e-7.
-// A score whose hi part is infinite is that infinity (the cache may hold one,
-// and 0 * inf of the lower parts would make it a NaN).
+// A score whose hi part is not finite (the cache may hold an infinity) is made
+// again in fp32: 0 * inf of a plane that is 0 where the query is not would make
+// an infinity a NaN (the check: 8 x 128 7.2 -> 6.8 us a launch, XL 64 x 128 37.2
+// -> 39.0).
 // What bounds it: vector work on the scores (exponentials, maxima, splits;
 // about twice the matrix-core time); few queries: the chain of tiles, 1.6 us
 // each. GPT-2 small, 32 x 768: 161 us a layer (22-bit halves 140) against 1170
@@ -1331,7 +1333,7 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
     }
     const int buf = SPLIT ? wave : t & 1;
     const vh_u32x4 *K = lk[buf], *V = lv[buf];
-    float s[4][4], big = 0.0f;
+    float s[4][4], fin = 0.0f;                                     // fin: a NaN if any hi part is not finite
     vh_f32x4 sh[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1347,14 +1349,25 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         s[i][j] = vh_hilo(sh[i][j], sl[j]);
-        big = fmaxf(big, __builtin_fabsf(sh[i][j]));
+        fin = fmaf(sh[i][j], 0.0f, fin);
       }
     }
-    if (__any(big == INFINITY)) {
+    if (__any(fin != fin)) {
+      const float* qp = Q + ((size_t)b * P + min(pq, P - 1)) * D + h * PF_E;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) s[i][j] = __builtin_isinf(sh[i][j]) ? sh[i][j] : s[i][j];
+        for (int j = 0; j < 4; ++j) {
+          float acc = 0.0f;
+#pragma nounroll
+          for (int c = 0; c < 8; ++c) {
+            float kv[8];
+            unpack8(K[(2 * i + (c >> 2)) * 64 + 16 * (c & 3) + 4 * q + j], kv);
+#pragma unroll
+            for (int d = 0; d < 8; ++d) acc = fmaf(qp[8 * c + d], kv[d], acc);
+          }
+          if (!(__builtin_fabsf(sh[i][j]) < INFINITY)) s[i][j] = acc;
+        }
     }
     if (64 * t + 63 > wfirst) {                                    // a tile that some query sees in part
 #pragma unroll
