@@ -70,3 +70,17 @@ def test_decode_attention_kernel_follows_the_block_count():
     src = prefill.prefill_source(448)
     for name in ('pf_attn1s', 'pf_mhead1', 'pf_mhead2', 'pf_mhead4'):
         assert f'void {name}(' in src or f'PF_MHEAD({name},' in src, name
+
+
+def test_lanes_that_share_lds_within_a_wave_order_their_accesses():
+    """The attention kernels' lanes hand each other values through LDS without a block barrier: the hardware executes a
+    wave's LDS operations in order, and ``pf_wave_sync`` on either side of each handover keeps the compiler to it."""
+    from vesta import prefill
+    src = prefill.prefill_source(448)
+    short = src[src.index('void pf_attn_short('):src.index('#define PF_SHORT')]
+    writes = [short.index('ws[s] = sc'), short.index('ws[lane] = ex / sum')]
+    reads = [short.index('expf(ws[lane]'), short.index('= ws[s]')]
+    syncs = [i for i in range(len(short)) if short.startswith('pf_wave_sync();', i)]
+    assert [sum(i < at for i in syncs) for at in (writes[0], reads[0], writes[1], reads[1])] == [1, 2, 2, 3]
+    split = src[src.index('if constexpr (SPLIT) {\n      pf_wave_sync();'):]
+    assert [ln.split(';')[0].strip() for ln in split.splitlines()[1:4]] == ['pf_wave_sync()', 'put(wave)', 'pf_wave_sync()']

@@ -1150,6 +1150,15 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_frag(const float* __
 // 8 x 128 7.5 (7.1) against 20.0; medium 3 x 333 after 100 positions 16.9 (15.0)
 // against 56.
 // F receives the head's output, row m, in fragment order.
+
+// A wave's lanes hand each other values through LDS, whose operations a wave
+// executes in order: this keeps the compiler to that order too (it emits
+// nothing).
+__device__ __forceinline__ void pf_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // One query over at most 64 positions by one wave, in fp32 throughout: eight
 // lanes per position for the dots (the partial dots added across them), a
 // lane per position for the weights, eight lanes of 8 dims for each residue of
@@ -1161,6 +1170,7 @@ __device__ __forceinline__ void pf_attn_short(const float* __restrict__ qp, cons
   float qv[8];
   pf_ld8f(qp + 8 * c8, qv);
   float mx = -INFINITY;
+  pf_wave_sync();                                                  // the query before is read
   for (int s = g; s <= pos; s += 8) {
     float kv[8], acc = 0.0f;
     unpack8(ld16(kb + (size_t)s * D + 8 * c8), kv);
@@ -1174,9 +1184,11 @@ __device__ __forceinline__ void pf_attn_short(const float* __restrict__ qp, cons
     mx = fmaxf(mx, sc);
   }
   mx = wave_red_max(mx);
+  pf_wave_sync();
   const float ex = lane <= pos ? expf(ws[lane] - mx) : 0.0f;
   const float sum = wave_red_sum(ex);
   ws[lane] = ex / sum;
+  pf_wave_sync();
 #pragma unroll
   for (int j = 0; j < 8; ++j) o[j] = 0.0f;
   for (int s = g; s <= pos; s += 8) {
@@ -1321,7 +1333,9 @@ __device__ __forceinline__ void pf_attn_body(const float* __restrict__ Q, const 
   }
   for (int t = SPLIT ? wave : 0; t < nt; t += SPLIT ? 4 : 1) {
     if constexpr (SPLIT) {
-      put(wave);                           // the wave's own tile: its LDS operations are in order
+      pf_wave_sync();                      // the wave's own tile: the one before is read
+      put(wave);
+      pf_wave_sync();
       if (t + 4 < nt) gload(t + 4);
     } else {
       vh_lds_sync();
