@@ -1,7 +1,7 @@
 """The products beyond 64 rows (hip/prefill.hip pf_pgemm*) on the GPU, each
 output tile forced in turn, against plain PyTorch in 64 bits: rows and
-columns at and around the edges of the tiles, each epilogue, split folds."""
-import numpy as np
+columns at and around the edges of the tiles, each epilogue, split folds; and
+the LayerNorms of many rows."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -42,6 +42,33 @@ def _close(got, want, bound):
     assert over <= 1, over
 
 
+def _exact(W, a, name, layer):
+    """The product, and its bound: 22-bit activations (2^-22 each) and K fp32 additions (2^-24 each) of terms whose
+    absolute values sum to s; plus rounding of the epilogue's few fp32 operations."""
+    w = W[name][layer].double()
+    s = a.double().abs() @ w.abs()
+    return a.double() @ w, s * (2.0 ** -22 + a.shape[1] * 2.0 ** -24)
+
+
+def _gelu(u):
+    """GELU in 64 bits, and its error per error of u (its slope is below 1.13; its exponential is good to 2^-20)."""
+    import torch
+    return 0.5 * u * (1 + torch.tanh(0.7978845608028654 * (u + 0.044715 * u ** 3))), 2.0 ** -20 * (u.abs() + 2.0 ** -10)
+
+
+def _check_cache(m, layer, t0, rows, P, want, bound):
+    """The cache rows of ``rows`` x P positions from t0 in fp16; those at or past the end are dropped, all others zero."""
+    import torch
+    n = max(0, min(P, m.tmax - t0))
+    for part, cache in ((1, m.keys), (2, m.vals)):
+        c = slice(part * D, (part + 1) * D)
+        w, b = (x.view(rows, P, -1)[:, :n, c] for x in (want, bound))
+        _close(cache[:rows, layer, t0:t0 + n].reshape(rows, n, D), w, b + 2.0 ** -11 * w.abs() + 2.0 ** -25)
+        rest = cache.clone()
+        rest[:rows, layer, t0:t0 + n] = 0
+        assert not rest.any()
+
+
 @pytest.mark.parametrize('kernel', ['pf_pgemm128', 'pf_pgemm64', 'pf_pgemm64w', 'pf_pgemm32'])
 @pytest.mark.parametrize('M', [65, 127, 128, 129, 257])
 def test_products_match_64_bits(engine, monkeypatch, kernel, M):
@@ -64,37 +91,29 @@ def test_products_match_64_bits(engine, monkeypatch, kernel, M):
         e.check()
 
     def exact(a, name):
-        """The product, and its bound: 22-bit activations (2^-22 each) and K fp32 additions (2^-24 each) of terms
-        whose absolute values sum to s; plus rounding of the epilogue's few fp32 operations."""
-        w = W[name][layer].double()
-        s = a.double().abs() @ w.abs()
-        return a.double() @ w, s * (2.0 ** -22 + a.shape[1] * 2.0 ** -24)
+        return _exact(W, a, name, layer)
 
     bias = {n: W[n][layer].double() for n in ('qkvb', 'ob', 'fcb', 'pb')}
-    # qkv: queries in fp32, cache rows (positions 7 .. 7 + P - 1, those at or past tmax dropped) in fp16
+    # qkv: queries in fp32, cache rows in fp16, all of them inside the cache and some past its end
+    for t0 in (7, TMAX - 60):
+        plan(1)
+        m.seek(t0)
+        m.keys.zero_(), m.vals.zero_()
+        Q = torch.empty(M, D, device='cuda')
+        e._pgemm(_frag(A), D, 'qkvw', layer, 3 * D, pf.MODE_QKV, bias=W['qkvb'][layer], out=Q, ldo=D, M=M, P=P)
+        run()
+        want, bound = exact(A, 'qkvw')
+        want, bound = want + bias['qkvb'], bound + 2.0 ** -23 * (want.abs() + 1)
+        _close(Q, want[:, :D], bound[:, :D])
+        _check_cache(m, layer, t0, 1, P, want, bound)
+    # GELU in fragment order (another 22-bit rounding)
     plan(1)
-    t0 = 7
-    m.seek(t0)
-    m.keys.zero_(), m.vals.zero_()
-    Q = torch.empty(M, D, device='cuda')
-    e._pgemm(_frag(A), D, 'qkvw', layer, 3 * D, pf.MODE_QKV, bias=W['qkvb'][layer], out=Q, ldo=D, M=M, P=P)
-    run()
-    want, bound = exact(A, 'qkvw')
-    want, bound = want + bias['qkvb'], bound + 2.0 ** -23 * (want.abs() + 1)
-    _close(Q, want[:, :D], bound[:, :D])
-    for n, cache in ((1, m.keys), (2, m.vals)):
-        c = slice(n * D, (n + 1) * D)
-        _close(cache[0, layer, t0:t0 + M].reshape(-1, D), want[:min(M, TMAX - t0), c],
-               bound[:TMAX - t0, c] + 2.0 ** -11 * want[:TMAX - t0, c].abs() + 2.0 ** -25)
-        assert not cache[0, layer, :t0].any() and not cache[0, layer, t0 + M:].any() and not cache[0, 0].any()
-    # GELU in fragment order (another 22-bit rounding; its slope is below 1.13 and its exponential good to 2^-20)
     out = torch.zeros(2 * 16 * pf._mtiles(M) * F, dtype=torch.float16, device='cuda')
     e._pgemm(_frag(A), D, 'fcw', layer, F, pf.MODE_GELU, bias=W['fcb'][layer], F=out, M=M)
     run()
     want, bound = exact(A, 'fcw')
-    u = want + bias['fcb']
-    want = 0.5 * u * (1 + torch.tanh(0.7978845608028654 * (u + 0.044715 * u ** 3)))
-    _close(_unfrag(out, M, F), want, 1.13 * bound + 2.0 ** -20 * (u.abs() + 2.0 ** -10))
+    want, own = _gelu(want + bias['fcb'])
+    _close(_unfrag(out, M, F), want, 1.13 * bound + own)
     # residual, whole and with a split fold whose parts the next LayerNorm's launch adds
     want, bound = exact(G, 'pw')
     want, bound = want + bias['pb'] + Z.double(), bound + 2.0 ** -22 * (want.abs() + Z.double().abs() + 1)
@@ -119,6 +138,51 @@ def test_products_match_64_bits(engine, monkeypatch, kernel, M):
     run()
     w = W['wte'].double()
     _close(out, A.double() @ w.t(), (A.double().abs() @ w.abs().t()) * (2.0 ** -22 + D * 2.0 ** -24))
+
+
+@pytest.fixture(scope='module')
+def engine3():
+    """Three batch rows, 24 layers: prompts of 2 to 8 tokens keep their order of sums."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip('no GPU')
+    from vesta.gpt2 import VestaGPT2
+    from vesta.weights import GPT2Shape, RandomGPT2
+    return VestaGPT2(RandomGPT2(GPT2Shape(24, D, 3, F, vocab=203), 7), batch=3, tmax=TMAX, engine='layered')
+
+
+@pytest.mark.parametrize('kernel', ['pf_mgemm', 'pf_pgemm128', 'pf_pgemm64', 'pf_pgemm64w', 'pf_pgemm32', 'pf_pgemm32o'])
+@pytest.mark.parametrize('P,t0', [(2, 5), (5, 298), (7, 0), (19, 290), (21, 40), (43, 270), (101, 3)])
+def test_new_cache_rows_go_to_their_batch_row_and_position(engine3, monkeypatch, kernel, P, t0):
+    """Three rows of prompt lengths that no tile divides, in tiled products of few rows too, whole and (pf_pgemm32o) with
+    the fold in parts that pf_reduce adds."""
+    import torch
+    from vesta import prefill as pf
+    m, M, layer = engine3, 3 * P, 5
+    e, W = m._pf, m.W
+    if kernel == 'pf_mgemm' and M > 64:
+        pytest.skip('products of up to 64 rows')
+    gen = torch.Generator(device='cuda').manual_seed(P)
+    A = torch.randn(M, D, generator=gen, device='cuda')
+    monkeypatch.setattr(pf, 'pgemm_plan', lambda *a: (kernel, 1))
+    want, bound = _exact(W, A, 'qkvw', layer)
+    want, bound = want + W['qkvb'][layer].double(), bound + 2.0 ** -23 * (want.abs() + 1)
+    for ks in (1, 2, 3) if kernel == 'pf_pgemm32o' else (None,):
+        m.seek(t0)
+        m.keys.zero_(), m.vals.zero_()
+        Q = torch.empty(M, D, device='cuda')
+        e._plan = []
+        kw = dict(bias=W['qkvb'][layer], out=Q, ldo=D, M=M, P=P)
+        if kernel == 'pf_mgemm':
+            e._mgemm(_frag(A), D, 'qkvw', layer, 3 * D, pf.MODE_QKV, **kw)
+        else:
+            e._pgemm(_frag(A), D, 'qkvw', layer, 3 * D, pf.MODE_QKV, ks=ks, **kw)
+        plan, e._plan = e._plan, []
+        assert plan[0][0].startswith(kernel)
+        e._replay(plan)
+        e.check()
+        _close(Q, want[:, :D], bound[:, :D])
+        _check_cache(m, layer, t0, 3, P, want, bound)
 
 
 @pytest.mark.parametrize('K,apart', [(1024, 1.57), (3072, 2.34)])
@@ -152,26 +216,35 @@ def test_a_long_fold_is_nearly_as_exact_as_a_short_one(engine, monkeypatch, K, a
 
 
 def test_more_than_64_rows_decode_and_prefill_like_fewer():
-    """70 rows (products in output tiles, the output head too) against the same rows in a batch of 8:
-    the same tokens where the margin is clear, logits within the engines' tolerance."""
+    """70 rows (products in output tiles, the output head too) against the same rows in a batch of 7, whose prompt goes a
+    step at a time (products of few rows): the same tokens where the margin is clear, logits within the engines'
+    tolerance."""
     import torch
     from vesta.gpt2 import VestaGPT2
     from vesta.weights import GPT2Shape, RandomGPT2, random_prompts
     hf = RandomGPT2(GPT2Shape(2, D, 3, F, vocab=203), 5)
     pr = torch.from_numpy(random_prompts(70, 9, 203, seed=3)).to('cuda', torch.int32)
+    seven = torch.arange(0, 70, 10, device='cuda') + 9
     got = []
-    for rows in (70, 8):
-        m = VestaGPT2(hf, batch=rows, tmax=32, engine='layered')
+    for rows in (torch.arange(70, device='cuda'), seven):
+        n = len(rows)
+        mine = slice(None) if n == 7 else seven
+        m = VestaGPT2(hf, batch=n, tmax=32, engine='layered')
         m.reset()
-        m.prefill(pr[:rows])
-        lg = [m.logits()[:8].clone()]
+        m.prefill(pr[rows].contiguous(), mode='batched' if n == 70 else 'steps')
+        lg, tok = [m.logits()[mine].clone()], [m.x[mine].clone()]
         for _ in range(3):
-            m.x.copy_(pr[:rows, 0])
+            m.x.copy_(pr[rows, 0])
             m.step()
-            lg.append(m.logits()[:8].clone())
+            lg.append(m.logits()[mine].clone())
+            tok.append(m.x[mine].clone())
         m.check()
-        got.append(torch.stack(lg).cpu().numpy())
-    assert np.abs(got[0] - got[1]).max() < 1e-3
+        got.append((torch.stack(lg), torch.stack(tok)))
+    (l70, t70), (l7, t7) = got
+    assert (l70 - l7).abs().max() < 1e-3
+    top = l7.topk(2, -1).values
+    clear = top[..., 0] - top[..., 1] > 2e-3
+    assert clear.sum() > 20 and torch.equal(t70[clear], t7[clear])
 
 
 @pytest.mark.parametrize('D', [64, 1024, 1088, 2048])
