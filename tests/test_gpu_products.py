@@ -185,6 +185,75 @@ def test_new_cache_rows_go_to_their_batch_row_and_position(engine3, monkeypatch,
         _check_cache(m, layer, t0, 3, P, want, bound)
 
 
+@pytest.mark.parametrize('M', [2, 8, 17, 33, 64, 130])
+def test_ordered_products_match_64_bits(engine, M):
+    """pf_pgemm32o at few rows, where it clamps its row tiles, its fold whole and in parts: GELU (parts added by
+    pf_reduce_frag), and the residual with the LayerNorm after it and without (pf_reduce_ln, pf_reduce)."""
+    import torch
+    from vesta import prefill as pf
+    m, e, layer = engine, engine._pf, 1
+    W = m.W
+    gen = torch.Generator(device='cuda').manual_seed(M)
+    A, G, Z = (torch.randn(M, n, generator=gen, device='cuda') for n in (D, F, D))
+
+    def run():
+        p, e._plan = e._plan, []
+        e._replay(p)
+        e.check()
+
+    for ks in (1, 2, 3):
+        out = torch.zeros(2 * 16 * pf._mtiles(M) * F, dtype=torch.float16, device='cuda')
+        e._plan = []
+        e._pgemm(_frag(A), D, 'fcw', layer, F, pf.MODE_GELU, bias=W['fcb'][layer], F=out, M=M, ks=ks)
+        run()
+        want, bound = _exact(W, A, 'fcw', layer)
+        want, own = _gelu(want + W['fcb'][layer].double())
+        _close(_unfrag(out, M, F), want, 1.13 * bound + own)
+        want, bound = _exact(W, G, 'pw', layer)
+        want, bound = want + W['pb'][layer].double() + Z.double(), bound + 2.0 ** -22 * (want.abs() + Z.double().abs() + 1)
+        for norm in (False, True):
+            z, nf = Z.clone(), torch.zeros(2 * 16 * pf._mtiles(M) * D, dtype=torch.float16, device='cuda')
+            done = e._pgemm(_frag(G), F, 'pw', layer, D, pf.MODE_RESID, bias=W['pb'][layer], out=z, ldo=D,
+                            ln=(W['ln1w'][layer], W['ln1b'][layer], nf) if norm else None, M=M, ks=ks)
+            run()
+            assert done == (norm and ks > 1)
+            _close(z, want, bound)
+            if done:
+                c = z.double() - z.double().mean(-1, keepdim=True)
+                y = c / torch.sqrt((c * c).mean(-1, keepdim=True) + 1e-5)      # gains 1, biases 0
+                _close(_unfrag(nf, M, D), y, 2.0 ** -18 * (y.abs() + 1))
+
+
+@pytest.mark.parametrize('P', [2, 5, 8, 9])
+@pytest.mark.parametrize('t0', [0, 6])
+def test_short_prompts_of_a_deep_model_match_single_steps(engine3, P, t0):
+    """24 layers, from an empty cache (up to 8 tokens: in the kept order of sums) and continued, against the same tokens
+    one decode step each: the same logits within the engines' tolerance, the same cache rows within fp16's rounding and
+    what it carries on (2^-9 of the largest value)."""
+    import torch
+    from vesta import prefill as pf
+    from vesta.weights import random_prompts
+    m = engine3
+    assert pf.ordered(P, m.L, t0) == (t0 == 0 and P <= 8)
+    pr = torch.from_numpy(random_prompts(3, 6 + P, 203, seed=P)).to('cuda', torch.int32)
+    got = []
+    for mode in ('batched', 'steps'):
+        m.reset()
+        if t0:
+            m.prefill(pr[:, :t0].contiguous(), mode='steps')
+        m.prefill(pr[:, t0:t0 + P].contiguous(), mode=mode)
+        m.check()
+        assert int(m.t) == t0 + P
+        got.append([x.float().clone() for x in (m.logits(), m.keys, m.vals)] + [m.x.clone()])
+    (lb, kb, vb, xb), (ls, ks, vs, xs) = got
+    assert (lb - ls).abs().max() < 1e-3
+    for a, b in ((kb, ks), (vb, vs)):
+        assert (a - b).abs().max() <= 2.0 ** -9 * b.abs().max()
+    top = ls.topk(2, -1).values
+    clear = top[:, 0] - top[:, 1] > 2e-3
+    assert clear.any() and torch.equal(xb[clear], xs[clear])
+
+
 @pytest.mark.parametrize('K,apart', [(1024, 1.57), (3072, 2.34)])
 def test_a_long_fold_is_nearly_as_exact_as_a_short_one(engine, monkeypatch, K, apart):
     """pf_pgemm32, which takes long folds whole at some hundred rows, sums 128 of them at a time. In rounding units, with

@@ -147,3 +147,29 @@ def test_mis_sized_tiled_products_are_refused(case):
     if case == 'fold':
         e._pgemm(**dict(kw, K=D))
         assert e._plan[0][0] in pf.PG_TILES
+
+
+@pytest.mark.parametrize('P,layers,t0,kept', [(1, 48, 0, False), (2, 48, 0, True), (8, 24, 0, True), (9, 48, 0, False),
+                                              (8, 23, 0, False), (2, 48, 1, False), (8, 48, 500, False)])
+def test_short_first_prompts_of_deep_models_keep_their_order_of_sums(P, layers, t0, kept):
+    """Only from an empty cache: a continued conversation takes the kernels its row count takes. The two ways of one
+    prompt length have plans of their own."""
+    assert pf.ordered(P, layers, t0) is kept
+    e = _engine()
+    built = []
+    e.m.L, e._plans, e._workspace, e._replay = layers, {}, lambda n: None, lambda plan: None
+    e._buffers = lambda M: dict(tok=torch.zeros(M, dtype=torch.int32))
+    e._build = lambda buf, B, P, tok, fixed: built.append(fixed)
+    for start in (t0, t0, 7):
+        e.run(torch.zeros(B, P, dtype=torch.int32), start)
+    assert built == ([True, False] if kept else [False])
+
+
+def test_an_ordered_product_splits_its_fold_by_the_rows_of_the_batch():
+    e = _engine()
+    e.fn.update({'pf_pgemm32o': None})
+    M, parts = 8, pf.ordered_parts(8, 4096, 1024)
+    assert parts == 4 and pf.ordered_parts(64, 4096, 1024) == 4 and pf.ordered_parts(65, 4096, 1024) == 3
+    e._pgemm(_af(M, F), F, 'pw', 0, D, pf.MODE_RESID, bias=torch.zeros(D), out=torch.zeros(M, D), ldo=D, M=M, ks=2)
+    assert [x[0] for x in e._plan] == ['pf_pgemm32o', 'pf_reduce']
+    assert e._plan[0][2] == 8 and e._plan[0][3].vals[5].value == 2     # one tile in two parts, eight XCDs

@@ -302,7 +302,7 @@ class VestaGPT2:
             if self._pf is None:
                 from .prefill import Prefill
                 self._pf = Prefill(self)
-            self._pf.run(prompt.to(dtype=self.x.dtype))
+            self._pf.run(prompt.to(dtype=self.x.dtype), t0)
             return
         ins = prompt.t().contiguous().to(dtype=self.x.dtype)
         if self.k is None:

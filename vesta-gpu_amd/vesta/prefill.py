@@ -119,22 +119,29 @@ def pgemm_plan(M, N, K, split):
                 or ks == 1), key=lambda c: pgemm_us(c[0], M, N, K, c[1]))
 
 
-def ordered(P, L):
-    """Whether a prompt of P tokens in a model of L layers goes through the
-    products and the attention whose order of sums is fixed by the model alone
-    (``ordered_parts``, ``pf_attn_short``). From an empty cache a short
-    prompt's attention averages over few positions, so a new cache row that
-    lies next to an fp16 rounding boundary and goes the other way is carried
-    on almost undiminished, layer after layer: with another order of sums,
-    XL's cache rows come out 1.9e-4 .. 2.8e-4 apart (2-norm) at 3-6 tokens,
-    2.1e-4 at 8, 1.6e-4 at 16; medium's 1.6e-4 .. 2.3e-4 at 3-4; GPT-2 small's
-    below 1.5e-4."""
-    return 1 < P <= ORDERED_TOKENS and L >= ORDERED_LAYERS
+def ordered(P, L, t0):
+    """Whether a prompt of P tokens at position t0 in a model of L layers keeps
+    the order of sums that prompts had in products of 64 x 64 tiles with split
+    folds and in an attention of one wave a query (``ordered_parts``,
+    ``pf_pgemm32o``, ``pf_attn_short``), so that its results stay the same bit
+    for bit. From an empty cache a short prompt's attention averages over few
+    positions, so a new cache row that lies next to an fp16 rounding boundary
+    and goes the other way is carried on almost undiminished, layer after
+    layer: with any other order of sums XL's cache rows come out 2.2e-4 ..
+    2.9e-4 apart (2-norm) at 2-6 tokens, about the 2.5e-4 by which
+    perf/cases.py lets results differ; 2.1e-4 at 8, 1.6e-4 at 16; after one
+    position 1.4e-4 .. 1.8e-4, after eight 0.8e-4; medium's 1.5e-4 .. 2.1e-4 at
+    2-8, GPT-2 small's below 1.5e-4. It is a matter of sameness alone: these
+    sums are no nearer to 64 bits (cache rows, XL 3 x 3 2.47e-4 against 2.44e-4,
+    3 x 7 2.19e-4 against 2.09e-4) and take longer (XL 4 x 3 2.54 ms against
+    2.07)."""
+    return t0 == 0 and 1 < P <= ORDERED_TOKENS and L >= ORDERED_LAYERS
 
 
 def ordered_parts(M, N, K):
     """Fold parts of an ordered product: about 384 output tiles of 64 x 64
-    times parts, each part at least 256 deep."""
+    times parts, each part at least 256 deep. (So the order is that of the
+    whole batch's size: the same for all batches of up to 64 rows in all.)"""
     return max(1, min(-(-384 // (-(-M // 64) * -(-N // 64))), K // 256))
 
 
@@ -405,14 +412,14 @@ class Prefill:
             self._grew = True
         return self._ws
 
-    def _plan_for(self, key, buf, B, P, tok):
+    def _plan_for(self, key, buf, B, P, tok, fixed=False):
         """The launch plan ``key``, built on first use (twice when the build
         grew the workspace, so that no launch keeps the old pointer)."""
         if key not in self._plans:
             self._workspace(1)
             for _ in range(2):
                 self._plan, self._grew = [], False
-                self._build(buf, B, P, tok)
+                self._build(buf, B, P, tok, fixed)
                 if not self._grew:
                     break
             self._plans[key] = self._plan
@@ -425,17 +432,20 @@ class Prefill:
         for name, fn, grid, a, block in plan:
             ok(L.vh_launch(fn, grid, block, 0, stream, a.array), name)
 
-    def run(self, prompt):
+    def run(self, prompt, t0=0):
         """Prefill ``prompt`` (int32 device tensor [B, P]) at positions t .. t + P - 1
-        (t the model's position counter, read and advanced on the device).
+        (t the model's position counter, read and advanced on the device;
+        ``t0``: the host's copy of it, for the choice of kernels alone).
 
         The launch sequence with its argument arrays is built once per P and
-        replayed: every pointer it holds (weights, cache, this object's
-        activation buffers and prompt copy) stays fixed."""
+        order of sums (``ordered``) and replayed: every pointer it holds
+        (weights, cache, this object's activation buffers and prompt copy)
+        stays fixed."""
         B, P = prompt.shape
         buf = self._buffers(B * P)
         buf['tok'].copy_(prompt.reshape(-1))
-        self._replay(self._plan_for(P, buf, B, P, buf['tok']))
+        fixed = ordered(P, self.m.L, t0)
+        self._replay(self._plan_for((P, fixed), buf, B, P, buf['tok'], fixed))
 
     def decode(self, n, tokens=None):
         """``n`` greedy decode steps, each one pass with P = 1 over the
@@ -475,11 +485,12 @@ class Prefill:
             self._replay(plan)
         return g
 
-    def _build(self, buf, B, P, tok):
+    def _build(self, buf, B, P, tok, fixed):
         """The launches of one pass: B rows of P positions each (P = 1: a
-        decode step). LayerNorm and attention write their outputs as the next
-        product's fragment-order activations (AF), the widening product its
-        GELU outputs as the narrowing one's (GF)."""
+        decode step; ``fixed``: the order of sums is kept, see ``ordered``).
+        LayerNorm and attention write their outputs as the next product's
+        fragment-order activations (AF), the widening product its GELU outputs
+        as the narrowing one's (GF)."""
         m = self.m
         M, D, H, L = B * P, m.D, m.H, m.L
         F = m.W['fcw'].shape[2]
@@ -487,7 +498,6 @@ class Prefill:
         W = m.W
         Z, Q, AF, GF, err = buf['Z'], buf['Q'], buf['AF'], buf['GF'], self.err
         mt = _mtiles(M)
-        fixed = ordered(P, L)
 
         def norm(w, b, to, rows, row0=0, stride=1):
             if rows >= LNM_ROWS and stride == 1:
