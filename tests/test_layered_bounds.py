@@ -157,7 +157,7 @@ def test_short_first_prompts_of_deep_models_keep_their_order_of_sums(P, layers, 
     assert pf.ordered(P, layers, t0) is kept
     e = _engine()
     built = []
-    e.m.L, e._plans, e._workspace, e._replay = layers, {}, lambda n: None, lambda plan: None
+    e.m.L, e._plans, e._replay = layers, {}, lambda plan: None
     e._buffers = lambda M: dict(tok=torch.zeros(M, dtype=torch.int32))
     e._build = lambda buf, B, P, tok, fixed: built.append(fixed)
     for start in (t0, t0, 7):
@@ -173,3 +173,30 @@ def test_an_ordered_product_splits_its_fold_by_the_rows_of_the_batch():
     e._pgemm(_af(M, F), F, 'pw', 0, D, pf.MODE_RESID, bias=torch.zeros(D), out=torch.zeros(M, D), ldo=D, M=M, ks=2)
     assert [x[0] for x in e._plan] == ['pf_pgemm32o', 'pf_reduce']
     assert e._plan[0][2] == 8 and e._plan[0][3].vals[5].value == 2     # one tile in two parts, eight XCDs
+
+
+def test_the_workspace_is_as_large_as_the_largest_split_product():
+    """A buffer that a later plan outgrows is replaced; launches recorded before follow it, and a captured graph, which
+    cannot, is dropped."""
+    e = _engine()
+    del e._workspace
+    e._ws, e._ws_at, e._graph = None, pf.ctypes.c_void_p(), 'captured'
+
+    def product(M):
+        e._plan = []
+        e._pgemm(_af(M, F), F, 'pw', 0, D, pf.MODE_RESID, bias=torch.zeros(D), out=torch.zeros(M, D), ldo=D, M=M, ks=2)
+        return [a.array for _, _, _, a, _ in e._plan]
+
+    def pointers(arrays):
+        at = [pf.ctypes.cast(x, pf.ctypes.POINTER(pf.ctypes.c_void_p)).contents.value
+              for x in (arrays[0][19], arrays[1][0])]
+        return at == [e._ws.data_ptr()] * 2
+    e.fn.update({'pf_pgemm32o': None})
+    small = product(8)
+    assert e._ws.numel() == 2 * 8 * D and pointers(small) and e._graph is None
+    e._graph = 'captured'
+    large = product(48)
+    assert e._ws.numel() == 2 * 48 * D and pointers(small) and pointers(large) and e._graph is None
+    e._graph = 'captured'
+    product(20)
+    assert e._ws.numel() == 2 * 48 * D and e._graph == 'captured'

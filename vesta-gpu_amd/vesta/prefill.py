@@ -55,7 +55,6 @@ MEM_CACHE_BYTES = 256 << 20   # the device's memory-side cache: decode products 
                               # larger load them nontemporal (same box: XL B=64 3.000 -> 2.944 ms per step,
                               # medium B=16 0.958 -> 0.916; GPT-2 small's 247 MB stay in that cache between
                               # steps, nontemporal there: 32 rows 0.548 -> 0.553)
-WORKSPACE_MIN = 8 << 20        # floats; a plan whose build outgrows the workspace is built twice (some ms of host time)
 LNM_ROWS = 1536               # LayerNorms of at least this many rows take a block per 16 rows (pf_lnm*; us a
                               # launch, block per row / per 16 rows: 999 x 768 6.3 / 7.3, 2048 x 768 8.7 / 7.7, 999 x
                               # 1600 8.3 / 12.7, 2048 x 1600 13.0 / 13.7, 4096 x 1600 24.0 / 15.9)
@@ -190,6 +189,9 @@ class _Args:
 
 
 def _p(t):
+    """A pointer argument: a tensor's, or one given as it is."""
+    if isinstance(t, ctypes.c_void_p):
+        return t
     return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
 
 
@@ -223,7 +225,7 @@ class Prefill:
         self._bufs = {}
         self._own = {}
         self._ws = None
-        self._grew = False
+        self._ws_at = ctypes.c_void_p()
         self._graph = None
         self._plans = {}
         self._plan = []
@@ -404,24 +406,21 @@ class Prefill:
 
     def _workspace(self, n):
         """Partial tiles of split products: one buffer, grown to the largest
-        need (launches on one stream run one after another)."""
+        need (launches on one stream run one after another). Returns the
+        argument that all launches share, which follows the buffer when it
+        grows."""
         import torch
         if self._ws is None or self._ws.numel() < n:
-            self._ws = torch.empty(max(n, WORKSPACE_MIN), dtype=torch.float32, device='cuda')
-            self._plans = {}            # plans hold the old pointer
-            self._grew = True
-        return self._ws
+            self._graph = None          # a captured graph holds the old pointer
+            self._ws = torch.empty(n, dtype=torch.float32, device=self.err.device)
+            self._ws_at.value = self._ws.data_ptr()
+        return self._ws_at
 
     def _plan_for(self, key, buf, B, P, tok, fixed=False):
-        """The launch plan ``key``, built on first use (twice when the build
-        grew the workspace, so that no launch keeps the old pointer)."""
+        """The launch plan ``key``, built on first use."""
         if key not in self._plans:
-            self._workspace(1)
-            for _ in range(2):
-                self._plan, self._grew = [], False
-                self._build(buf, B, P, tok, fixed)
-                if not self._grew:
-                    break
+            self._plan = []
+            self._build(buf, B, P, tok, fixed)
             self._plans[key] = self._plan
         return self._plans[key]
 
