@@ -200,3 +200,21 @@ def test_the_workspace_is_as_large_as_the_largest_split_product():
     e._graph = 'captured'
     product(20)
     assert e._ws.numel() == 2 * 48 * D and e._graph == 'captured'
+
+
+@pytest.mark.parametrize('tiled', [False, True])
+def test_products_without_a_kernel_for_them_are_refused(tiled):
+    """A plain product in parts, or of few rows (the output head has its own kernels), and a residual whose LayerNorm
+    would read rows of another pitch."""
+    e = _engine()
+    e.fn.update({n: None for n in ('pf_pgemm32o', *pf.PG_TILES)})
+    M = 70 if tiled else B
+    product = e._pgemm if tiled else e._mgemm
+    a = (_af(M, D), D, 'ow', 0, D)
+    more = dict(ks=2) if tiled else {}
+    with pytest.raises(ValueError, match='whole|pf_mhead'):
+        product(*a, pf.MODE_PLAIN, out=torch.zeros(M, D), ldo=D, M=M, **more)
+    ln = (torch.zeros(D), torch.zeros(D), _af(M, D))
+    with pytest.raises(ValueError, match='pitch'):
+        product(*a, pf.MODE_RESID, bias=torch.zeros(D), out=torch.zeros(M, 2 * D), ldo=2 * D, M=M, ln=ln)
+    assert e._plan == []

@@ -149,7 +149,7 @@ class VestaGPT2:
             from .prefill import Prefill
             if not supported(D, H, F):
                 raise ValueError(f'the persistent kernel does not fit ({self.why_layered}) and the layered '
-                                 f'engine needs 64-wide heads and widths that are multiples of 32')
+                                 f'engine needs 64-wide heads and widths that are multiples of 64')
             self.engine = 'layered'
             self._logit = torch.zeros(batch, V, dtype=torch.float32, device='cuda')
             self._next = torch.zeros(batch, dtype=torch.float32, device='cuda')
@@ -290,7 +290,7 @@ class VestaGPT2:
         fits = supported(self.D, self.H, self.W['fcw'].shape[2])
         if mode == 'batched' and (tokens is not None or not fits):
             raise ValueError('batched prefill writes no per-step tokens and needs 64-wide heads and widths '
-                             'that are multiples of 32')
+                             'that are multiples of 64')
         if tokens is not None and not (tokens.is_cuda and tokens.dtype == self.x.dtype and tokens.is_contiguous()
                                        and tokens.numel() >= P * self.B):
             raise TypeError(f'tokens must be a contiguous int32 device tensor of at least {P * self.B} ids')

@@ -103,15 +103,13 @@ __device__ __forceinline__ float pf_gelu(float u) {
   return u / (1.0f + __expf(-2.0f * y));
 }
 
-// The epilogue of one output value c = C[m, n] (modes 0, 1 and 3).
+// The epilogue of one output value c = C[m, n] (modes 1 and 3).
 __device__ __forceinline__ void pf_epi(int mode, int m, int n, float c, const vh_half* __restrict__ bias, int N,
                                        float* __restrict__ out, int ldo, vh_half* __restrict__ kc,
                                        vh_half* __restrict__ vc, int P, const int* __restrict__ tp, int layer,
                                        int L, int tmax) {
   const float bn = bias ? h2f(bias[n]) : 0.0f;
-  if (mode == 0) {
-    out[(size_t)m * ldo + n] = c + bn;
-  } else if (mode == 1) {
+  if (mode == 1) {
     float* o = out + (size_t)m * ldo + n;
     *o = (*o + c) + bn;
   } else {
@@ -144,7 +142,7 @@ __device__ __forceinline__ void pf_epi(int mode, int m, int n, float c, const vh
 // converted fp32 activations in every block took 380. With few tiles a CU it
 // is the tile's fixed part (first loads, epilogue: 4-8 us).
 // `ks` > 1 splits the fold over blocks: part p of tile t stores its sums in
-// ws[p][m][n] for pf_reduce_ln.
+// ws[p][m][n] for pf_reduce_ln, pf_reduce or pf_reduce_frag.
 //
 // Tiles go to the 8 XCDs (blockIdx % 8) in contiguous runs, within a run in
 // groups of 4 row tiles, so that the blocks resident on one XCD share their
@@ -285,17 +283,17 @@ __device__ __forceinline__ void pf_pgemm_out(
   }
 }
 
-// Ring: NR stages of S k-steps of 32 in flight in registers before they go to
+// Ring: two stages of S k-steps of 32 in flight in registers before they go to
 // LDS; with WDIR the weight fragments skip LDS and go from the caches straight
 // into each wave's registers one stage ahead (the WM waves that share them
 // meet in the CU's L1). With ANEW the hi halves' sums start anew with each turn
-// of the loop (NR stages) and are added in fp32: a fold in one running sum is up
+// of the loop (two stages) and are added in fp32: a fold in one running sum is up
 // to 1.7 times further from 64 bits than in parts of 256, which is what few rows
 // get from the waves and the blocks that split their folds (pf_pgemm32, 128
 // rows, in one sum / anew every 128: 1024 deep 2.10e-7 / 1.08e-7). It costs 0-1%
 // (1024 x 2304 x 768 17.9 -> 18.0 us); sums twice as long, behind a condition,
 // 2%.
-template <int TM, int TN, int WM, int WN, int S, bool WDIR, int NR, bool ANEW>
+template <int TM, int TN, int WM, int WN, int S, bool WDIR, bool ANEW>
 __device__ __forceinline__ void pf_pgemm_ring(
     const vh_u32x4* __restrict__ Af, const vh_u32x4* __restrict__ Wf, int MT, int KT, int NT, int ks,
     const vh_half* __restrict__ bias, int M, int N, int mode, float* __restrict__ out, int ldo,
@@ -304,7 +302,7 @@ __device__ __forceinline__ void pf_pgemm_ring(
   constexpr int NW = WM * WN, BM = TM * WM, BN = TN * WN;
   constexpr int FA = 2 * BM * S, FR = FA + (WDIR ? 0 : BN * S);     // fragments (1 KB) of a stage: A, all
   constexpr int PER = FR / NW;
-  static_assert(FR % NW == 0 && (NR == 1 || NR % 2 == 0), "whole fragments per wave; stages alternate two buffers");
+  static_assert(FR % NW == 0, "whole fragments per wave");
   __shared__ __attribute__((aligned(16))) vh_u32x4 lds[2][FR * 64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = wave / WN, wn = wave % WN;
@@ -330,7 +328,7 @@ __device__ __forceinline__ void pf_pgemm_ring(
   for (int a = 0; a < TM; ++a)
 #pragma unroll
     for (int b = 0; b < TN; ++b) ah[a][b] = al[a][b] = sum[a][b] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  vh_u32x4 st[NR][PER];
+  vh_u32x4 st[2][PER];
   auto gload = [&](vh_u32x4 (&d)[PER], int c) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) d[i] = src[i][(size_t)c * S * 64];
@@ -352,18 +350,17 @@ __device__ __forceinline__ void pf_pgemm_ring(
   }
   put(st[0], 0);
 #pragma unroll
-  for (int u = 1; u <= NR; ++u)
-    if (u < ns) gload(st[u % NR], u);
+  for (int u = 1; u <= 2; ++u)
+    if (u < ns) gload(st[u % 2], u);
   vh_lds_sync();
-  constexpr int U = NR == 1 ? 2 : NR;
-  for (int cc = 0; cc < ns; cc += U) {
+  for (int cc = 0; cc < ns; cc += 2) {
     if constexpr (ANEW)
 #pragma unroll
       for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int b = 0; b < TN; ++b) ah[a][b] = vh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < 2; ++u) {
       const int c = cc + u;
       if (c >= ns) break;
       const vh_u32x4* sh = lds[u & 1];
@@ -394,8 +391,8 @@ __device__ __forceinline__ void pf_pgemm_ring(
             for (int b = 0; b < TN; ++b) wd[s][b] = wp[b][(size_t)((c + 1) * S + s) * 64];
       }
       if (c + 1 < ns) {       // the buffer written here was last read before the previous barrier
-        put(st[(u + 1) % NR], (u + 1) & 1);
-        if (c + 1 + NR < ns) gload(st[(u + 1) % NR], c + 1 + NR);
+        put(st[u ^ 1], u ^ 1);
+        if (c + 3 < ns) gload(st[u ^ 1], c + 3);
       }
       vh_lds_sync();
     }
@@ -526,9 +523,9 @@ __device__ __forceinline__ void pf_pgemm_pipe(
   }
 PF_PGEMM(pf_pgemm128, 512, 2, pf_pgemm_pipe<4, 4, 2, 4>)              // 128 x 256
 PF_PGEMM(pf_pgemm64, 512, 4, pf_pgemm_pipe<2, 2, 2, 4>)               // 64 x 128, eight waves
-PF_PGEMM(pf_pgemm64w, 256, 2, pf_pgemm_ring<2, 4, 2, 2, 1, true, 2, false>)  // 64 x 128, four waves
-PF_PGEMM(pf_pgemm32, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, 2, true>)   // 32 x 64
-PF_PGEMM(pf_pgemm32o, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, 2, false>) // 32 x 64, one sum a part
+PF_PGEMM(pf_pgemm64w, 256, 2, pf_pgemm_ring<2, 4, 2, 2, 1, true, false>)  // 64 x 128, four waves
+PF_PGEMM(pf_pgemm32, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, true>)   // 32 x 64
+PF_PGEMM(pf_pgemm32o, 256, 2, pf_pgemm_ring<1, 2, 2, 2, 2, false, false>) // 32 x 64, one sum a part
 
 // The parts of a split product added in part order, then the epilogue. One
 // thread per output value.
@@ -770,7 +767,7 @@ PF_LNM(pf_lnm16, 16)
 // next k-step's weights and activations in flight. The waves' partial tiles
 // are added in LDS in wave order. Then either the part is stored (ks > 1:
 // ws[part][m][n], added by pf_reduce / pf_reduce_ln / pf_reduce_frag), or the
-// epilogue of `mode` is applied: 0, 1 and 3 as pf_epi;
+// epilogue of `mode` is applied: 1 and 3 as pf_epi;
 // 2 (GELU) writes the result in fragment order into F, as the activation of
 // the next product (N / 32 k-steps).
 #define PF_MW 8
@@ -980,27 +977,19 @@ __device__ __forceinline__ void pf_mgemm_body(
     if (bad) stc_u(err, VH_ERR_RANGE);
     return;
   }
-  if (ks > 1 || mode == 1 || mode == 3) {   // eight consecutive columns per thread, 16-byte stores
-    for (int e = threadIdx.x; e < 16 * MT * 2 * MN; e += PF_MW * 64) {
-      const int m = e / (2 * MN), c8 = 8 * (e % (2 * MN)), n = n0 + c8;
-      if (m >= M || n >= N) continue;
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = tile[m][c8 + j];
-      if (ks > 1) {
-        float* p = ws + ((size_t)part * M + m) * N + n;
-        *(vh_f32x4*)p = vh_f32x4{v[0], v[1], v[2], v[3]};
-        *(vh_f32x4*)(p + 4) = vh_f32x4{v[4], v[5], v[6], v[7]};
-      } else {
-        pf_epi8(mode, m, n, v, eb, ez, epos, N, out, ldo, kc, vc, P, layer, L, tmax);     // (e is this thread's item)
-      }
-    }
-    return;
-  }
-  for (int e = threadIdx.x; e < 16 * MT * 16 * MN; e += PF_MW * 64) {
-    const int m = e / (16 * MN), c = e % (16 * MN), n = n0 + c;
+  for (int e = threadIdx.x; e < 16 * MT * 2 * MN; e += PF_MW * 64) {   // eight consecutive columns per thread, 16-byte stores
+    const int m = e / (2 * MN), c8 = 8 * (e % (2 * MN)), n = n0 + c8;
     if (m >= M || n >= N) continue;
-    pf_epi(mode, m, n, tile[m][c], bias, N, out, ldo, kc, vc, P, tp, layer, L, tmax);
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = tile[m][c8 + j];
+    if (ks > 1) {
+      float* p = ws + ((size_t)part * M + m) * N + n;
+      *(vh_f32x4*)p = vh_f32x4{v[0], v[1], v[2], v[3]};
+      *(vh_f32x4*)(p + 4) = vh_f32x4{v[4], v[5], v[6], v[7]};
+    } else {
+      pf_epi8(mode, m, n, v, eb, ez, epos, N, out, ldo, kc, vc, P, layer, L, tmax);     // (e is this thread's item)
+    }
   }
 }
 

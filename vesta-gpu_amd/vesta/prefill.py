@@ -34,10 +34,10 @@ PRELUDE_SRC = Path(__file__).resolve().parent / 'hip' / 'prelude.h'
 BLOCK = 256
 CHUNK = 64                    # products' fold lengths are multiples of this (two 32-deep k-steps)
 HEAD = 64
-KERNELS = ('pf_ln', 'pf_lnm8', 'pf_lnm16', 'pf_reduce', 'pf_reduce_ln', 'pf_attn', 'pf_attn16', 'pf_attn1', 'pf_argmax_part', 'pf_argmax',
-           'pf_mgemm1', 'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n', 'pf_mgemm2n', 'pf_mgemm4n', 'pf_reduce_frag', 'pf_attn1s',
-           'pf_mhead1', 'pf_mhead2', 'pf_mhead4', 'pf_embed_ln', 'pf_pgemm128', 'pf_pgemm64',
-           'pf_pgemm64w', 'pf_pgemm32', 'pf_pgemm32o')
+KERNELS = ('pf_embed_ln', 'pf_ln', 'pf_lnm8', 'pf_lnm16', 'pf_mgemm1', 'pf_mgemm2', 'pf_mgemm4', 'pf_mgemm1n',
+           'pf_mgemm2n', 'pf_mgemm4n', 'pf_pgemm128', 'pf_pgemm64', 'pf_pgemm64w', 'pf_pgemm32', 'pf_pgemm32o',
+           'pf_reduce', 'pf_reduce_ln', 'pf_reduce_frag', 'pf_attn', 'pf_attn16', 'pf_attn1', 'pf_attn1s', 'pf_mhead1',
+           'pf_mhead2', 'pf_mhead4', 'pf_argmax_part', 'pf_argmax')
 ARGMAX_SPLIT = 32             # blocks per row of the output-head argmax (same box, 16 -> 32: GPT-2 small 32 rows
                               # 547.6 -> 545.8 us per step, 8 rows 396.3 -> 395.5, XL 64 rows even)
 # output tiles of the products beyond FEW_ROWS rows: 16-row tiles, 16-column tiles and waves of a block
@@ -206,7 +206,7 @@ class Prefill:
         self.m = model
         self.graphs = graphs           # layered decode steps replay a captured HIP graph
         if not supported(model.D, model.H, model.W['fcw'].shape[2]):
-            raise ValueError(f'prefill kernels need 64-wide heads and widths that are multiples of 32 '
+            raise ValueError(f'prefill kernels need 64-wide heads and widths that are multiples of 64 '
                              f'(d={model.D}, H={model.H})')
         self.code = compile_code(prefill_source(model.tmax))
         L = lib()
@@ -289,9 +289,9 @@ class Prefill:
         return self._own[key]
 
     def _mgemm(self, Af, K, wname, layer, N, mode, bias=None, out=None, ldo=0, F=None, ln=None, M=1, P=1):
-        """One product of at most 64 rows (``pf_mgemm*``) over M rows (P positions each of M / P rows): A in fragment order
-        (Af), weights ``wname`` (layer ``layer``) in fragment order. With a
-        split fold the parts are added by a second launch: ``pf_reduce_ln``
+        """One product of at most 64 rows (``pf_mgemm*``) over M rows (P
+        positions each of M / P rows): A in fragment order (Af), weights
+        ``wname`` (layer ``layer``) in fragment order. With a split fold the parts are added by a second launch: ``pf_reduce_ln``
         for a residual product followed by the LayerNorm ``ln`` = (w, b, F_out)
         (returns True: that LayerNorm is done), ``pf_reduce_frag`` for the
         GELU product, ``pf_reduce`` otherwise."""
@@ -299,7 +299,7 @@ class Prefill:
         KT, NT = K // 32, -(-N // 16)
         mt = _mtiles(M)
         if K % 32 or M > 16 * mt or mt > 4:
-            raise ValueError(f'decode product: K={K} must be a multiple of 32 and M={M} at most 64')
+            raise ValueError(f'product {wname}: K={K} must be a multiple of 32 and M={M} at most 64')
         nb = -(-NT // MG_TILES[mt])
         steps = MG_MIN_STEPS_LN if mode == MODE_RESID and ln is not None else MG_MIN_STEPS
         ks = max(1, min(round(MG_BLOCKS / nb), KT // steps))
@@ -308,11 +308,15 @@ class Prefill:
         Wf = Wf[layer] if layer is not None else Wf
         # the extents pf_mgemm* indexes, checked before the launch is recorded
         if Af.numel() < 2 * 16 * mt * K or Wf.numel() < NT * KT * 512:
-            raise ValueError(f'decode product {wname}: operands smaller than {M}x{K} activations / {N}x{K} weights')
+            raise ValueError(f'product {wname}: operands smaller than {M}x{K} activations / {N}x{K} weights')
         if mode == MODE_GELU and (N % 32 or F is None or F.numel() < 2 * 16 * mt * N):
-            raise ValueError(f'decode product {wname}: GELU output needs a fragment buffer of {M}x{N}, N % 32 == 0')
-        if mode in (MODE_PLAIN, MODE_RESID, MODE_QKV) and out.numel() < M * ldo:
-            raise ValueError(f'decode product {wname}: output smaller than {M} rows of {ldo}')
+            raise ValueError(f'product {wname}: GELU output needs a fragment buffer of {M}x{N}, N % 32 == 0')
+        if mode == MODE_PLAIN:
+            raise ValueError(f'product {wname}: the output head of up to 64 rows is pf_mhead*')
+        if mode == MODE_RESID and ln is not None and ldo != N:
+            raise ValueError(f'product {wname}: a LayerNorm over rows of {N} needs their pitch to be {N}')
+        if mode != MODE_GELU and out.numel() < M * ldo:
+            raise ValueError(f'product {wname}: output smaller than {M} rows of {ldo}')
         t_args = [_p(m.keys), _p(m.vals), _i(P), _p(m.t), _i(layer or 0), _i(m.L), _i(m.tmax)]
         self._launch(f'pf_mgemm{mt}' + ('n' if self._weights_nt() else ''), nb * ks,
                      [_p(Af), _p(Wf), _i(KT), _i(NT), _i(ks), _p(bias), _i(M), _i(N), _i(mode), _p(out), _i(ldo)]
@@ -327,7 +331,7 @@ class Prefill:
         m = self.m
         KT, NT, MT = K // 32, -(-N // 16), _mtiles(M)
         if ks is None:
-            name, ks = pgemm_plan(M, N, K, mode == MODE_RESID and ln is not None and ldo == N)
+            name, ks = pgemm_plan(M, N, K, mode == MODE_RESID and ln is not None)
             bm, bn, waves = PG_TILES[name]
         else:
             name, (bm, bn, waves) = 'pf_pgemm32o', PG_TILES['pf_pgemm32']
@@ -343,6 +347,10 @@ class Prefill:
             raise ValueError(f'product {wname}: GELU output needs a fragment buffer of {M}x{N}, N % 32 == 0')
         if mode != MODE_GELU and out.numel() < (M - 1) * ldo + (N // 3 if mode == MODE_QKV else N):
             raise ValueError(f'product {wname}: output smaller than {M} rows of {ldo}')
+        if mode == MODE_PLAIN and ks > 1:
+            raise ValueError(f'product {wname}: a plain product is made whole')
+        if mode == MODE_RESID and ln is not None and ldo != N:
+            raise ValueError(f'product {wname}: a LayerNorm over rows of {N} needs their pitch to be {N}')
         if mode != MODE_PLAIN and (N % 64 or ldo % 4 or bias is None):
             raise ValueError(f'product {wname}: N={N} must be a multiple of 64, the output pitch of 4, with a bias')
         tiles = -(-MT // bm) * -(-NT // bn) * ks
