@@ -416,3 +416,27 @@ def test_layer_norm_of_many_rows_takes_what_of_few_takes(engine, D, size):
     many, few = _lnm_and_ln(engine._pf, X, w.half(), b.half())
     engine.check()
     _close(many, few, (2.0 ** -20 + D ** 0.5 * 2.0 ** -23) * (many.abs() + few.abs() + 1))
+
+
+def test_a_prompt_of_many_rows_matches_its_rows_alone():
+    """1600 rows of activations (LayerNorms of 16 rows a block, from the batched pass itself) against two of its batch
+    rows in a model of their own, 400 rows (a block per row): the same cache rows within fp16's rounding and what it
+    carries on (2^-9 of the largest value), logits within the engines' tolerance."""
+    import torch
+    from vesta import prefill as pf
+    from vesta.gpt2 import VestaGPT2
+    from vesta.weights import GPT2Shape, RandomGPT2, random_prompts
+    hf = RandomGPT2(GPT2Shape(2, D, 3, F, vocab=203), 8)
+    pr = torch.from_numpy(random_prompts(8, 200, 203, seed=9)).to('cuda', torch.int32)
+    got = []
+    for rows in ([0, 1, 2, 3, 4, 5, 6, 7], [2, 7]):
+        m = VestaGPT2(hf, batch=len(rows), tmax=208, engine='layered')
+        m.prefill(pr[rows].contiguous())
+        m.check()
+        names = {x[0] for x in m._pf._plans[200, False]}
+        assert ('pf_lnm8' in names) == (len(rows) * 200 >= pf.LNM_ROWS)
+        mine = [2, 7] if len(rows) == 8 else [0, 1]
+        got.append([x[mine].float() for x in (m.logits(), m.keys, m.vals)])
+    assert (got[0][0] - got[1][0]).abs().max() < 1e-3
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert (a - b).abs().max() <= 2.0 ** -9 * b.abs().max()
