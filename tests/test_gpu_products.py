@@ -151,8 +151,9 @@ def engine3():
     return VestaGPT2(RandomGPT2(GPT2Shape(24, D, 3, F, vocab=203), 7), batch=3, tmax=TMAX, engine='layered')
 
 
-@pytest.mark.parametrize('kernel', ['pf_mgemm', 'pf_pgemm128', 'pf_pgemm64', 'pf_pgemm64w', 'pf_pgemm32', 'pf_pgemm32o'])
-@pytest.mark.parametrize('P,t0', [(2, 5), (5, 298), (7, 0), (19, 290), (21, 40), (43, 270), (101, 3)])
+@pytest.mark.parametrize('kernel,P,t0', [
+    (k, P, t0) for k in ('pf_mgemm', 'pf_pgemm128', 'pf_pgemm64', 'pf_pgemm64w', 'pf_pgemm32', 'pf_pgemm32o')
+    for P, t0 in ((2, 5), (5, 298), (7, 0), (19, 290), (21, 40), (43, 270), (101, 3)) if k != 'pf_mgemm' or 3 * P <= 64])
 def test_new_cache_rows_go_to_their_batch_row_and_position(engine3, monkeypatch, kernel, P, t0):
     """Three rows of prompt lengths that no tile divides, in tiled products of few rows too, whole and (pf_pgemm32o) with
     the fold in parts that pf_reduce adds."""
@@ -160,8 +161,6 @@ def test_new_cache_rows_go_to_their_batch_row_and_position(engine3, monkeypatch,
     from vesta import prefill as pf
     m, M, layer = engine3, 3 * P, 5
     e, W = m._pf, m.W
-    if kernel == 'pf_mgemm' and M > 64:
-        pytest.skip('products of up to 64 rows')
     gen = torch.Generator(device='cuda').manual_seed(P)
     A = torch.randn(M, D, generator=gen, device='cuda')
     monkeypatch.setattr(pf, 'pgemm_plan', lambda *a: (kernel, 1))

@@ -1130,14 +1130,15 @@ extern "C" __global__ __launch_bounds__(256) void pf_reduce_frag(const float* __
 // 1.33e-7 / 1.50e-7 / 1.08e-7.
 // A score whose hi part is not finite (the cache may hold an infinity) is made
 // again in fp32: 0 * inf of a plane that is 0 where the query is not would make
-// an infinity a NaN (the check: 8 x 128 7.2 -> 6.8 us a launch, XL 64 x 128 37.2
-// -> 39.0).
+// an infinity a NaN.
 // What bounds it: vector work on the scores (exponentials, maxima, splits;
 // about twice the matrix-core time); few queries: the chain of tiles, 1.6 us
-// each. GPT-2 small, 32 x 768: 161 us a layer (22-bit halves 140) against 1170
-// with a wave per (query row, head), which read every cache row once per query;
-// 8 x 128 7.5 (7.1) against 20.0; medium 3 x 333 after 100 positions 16.9 (15.0)
-// against 56.
+// each. GPT-2 small, 32 x 768: 144 us a layer alone and 153 in a pass, against
+// 1198 with a wave per (query row, head), which read every cache row once per
+// query; 8 x 128 6.8 against 19.7; medium 3 x 333 after 100 positions 16.5 alone
+// and 18 in a pass against 59. The third plane and the sums by tile are 6-15% of
+// that (32 x 768 140 -> 161 on one box, 8 x 128 7.1 -> 7.5), the check for scores
+// that are not finite -5 to 5% (8 x 128 7.2 -> 6.8, XL 64 x 128 37.2 -> 39.0).
 // F receives the head's output, row m, in fragment order.
 
 // A wave's lanes hand each other values through LDS, whose operations a wave
